@@ -1624,36 +1624,18 @@ void weight_vjp(nnpx_ctx* c, int precision, const double* u, const double* cE, d
         timed(c, "tangent32", [&] { launch_tangent32(c->mixed, t, c->d_model, s, u, Gdot, ldG, c->stream); });
     }
     GradArgs a{};
-    int total = 0;
-    for (int e = 0; e < t.nelem; ++e) {
-        a.coff[e] = total;
-        a.nconn[e] = num_connections(t.el[e].nn);
-        a.nconn_max = std::max(a.nconn_max, a.nconn[e]);
-        total += a.nconn[e];
-    }
+    const int blocks = plan_grad(a, t, c->elem_count.data(), c->elem_off.data(), c->mixed.tune.grad_atoms);
+    if (grad_act_bytes(a, precision == NNPX_MIXED) > 65536)
+        fail(NNPX_ERR_UNSUPPORTED, "network too wide for the gradient kernel's LDS staging");
     a.w = c->d_w;
-    a.nweights = t.nweights;
     a.G = existing<double>(c, "G");
     a.Gdot = Gdot;
-    a.ldG = ldG;
     a.cE = cE;
     a.sid = existing<int>(c, "sid");
     a.atoms = existing<int>(c, "elem_atoms");
-    a.nelem = t.nelem;
-    a.maxw = std::max(t.max_width, t.max_sf);
-    a.per_block = c->mixed.tune.grad_atoms;
     a.grad = gd;
     a.ldgrad = ldgrad;
-    int blocks = 0;
-    for (int e = 0; e < t.nelem; ++e) {
-        a.blk_off[e] = blocks;
-        a.atom_off[e] = c->elem_off[e];
-        blocks += (c->elem_count[e] + a.per_block - 1) / a.per_block;
-    }
-    a.blk_off[t.nelem] = blocks;
-    a.atom_off[t.nelem] = c->elem_off[t.nelem];
-    if (grad_act_bytes(a, precision == NNPX_MIXED) > 65536)
-        fail(NNPX_ERR_UNSUPPORTED, "network too wide for the gradient kernel's LDS staging");
+    if (ldgrad == 0) a.part = buf<double>(c, "t_part", (size_t)blocks * a.nconn_max);
     timed(c, precision == NNPX_MIXED ? "grad32" : "grad64",
           [&] { launch_grad(c->d_model, a, blocks, precision == NNPX_MIXED, c->stream); });
 }
@@ -2066,46 +2048,27 @@ nnpx_status nnpx_autotune(nnpx_ctx* c)
             // atoms per block of the gradient kernel (FP32 network pass on the
             // current G with a zero tangent)
             GradArgs a{};
-            int total = 0;
-            for (int e = 0; e < t.nelem; ++e) {
-                a.coff[e] = total;
-                a.nconn[e] = num_connections(t.el[e].nn);
-                a.nconn_max = std::max(a.nconn_max, a.nconn[e]);
-                total += a.nconn[e];
-            }
             double* cE = buf<double>(c, "t_cE", c->S);
-            double* gd = buf<double>(c, "t_grad", total);
+            double* gd = buf<double>(c, "t_grad", total_connections(t));
             hip_check(hipMemsetAsync(cE, 0, sizeof(double) * c->S, c->stream), "hipMemsetAsync");
             hip_check(hipMemsetAsync(Gdot, 0, sizeof(double) * (size_t)c->N * ldG, c->stream), "hipMemsetAsync");
             a.w = c->d_w;
-            a.nweights = t.nweights;
             a.G = existing<double>(c, "G");
             a.Gdot = Gdot;
-            a.ldG = ldG;
             a.cE = cE;
             a.sid = existing<int>(c, "sid");
             a.atoms = existing<int>(c, "elem_atoms");
-            a.nelem = t.nelem;
-            a.maxw = std::max(t.max_width, t.max_sf);
             a.grad = gd;
             double best_g = 1e30;
-            if (grad_lds_bytes(a, true) <= 65536) {
-                for (int per : {8, 16, 32, 64, 128}) {
-                    a.per_block = per;
-                    int blocks = 0;
-                    for (int e = 0; e < t.nelem; ++e) {
-                        a.blk_off[e] = blocks;
-                        a.atom_off[e] = c->elem_off[e];
-                        blocks += (c->elem_count[e] + per - 1) / per;
-                    }
-                    a.blk_off[t.nelem] = blocks;
-                    a.atom_off[t.nelem] = c->elem_off[t.nelem];
-                    c->ktime.clear();
-                    launch_grad(c->d_model, a, blocks, true, c->stream);
-                    for (int r = 0; r < 3; ++r) timed(c, "grad32", [&] { launch_grad(c->d_model, a, blocks, true, c->stream); });
-                    const double g = mean_time(c, "grad32");
-                    if (g < best_g) { best_g = g; tu.grad_atoms = per; }
-                }
+            for (int per : {8, 16, 32, 64, 128}) {
+                const int blocks = plan_grad(a, t, c->elem_count.data(), c->elem_off.data(), per);
+                if (grad_act_bytes(a, true) > 65536) break;  // no gradients for networks this wide
+                a.part = buf<double>(c, "t_part", (size_t)blocks * a.nconn_max);
+                c->ktime.clear();
+                launch_grad(c->d_model, a, blocks, true, c->stream);
+                for (int r = 0; r < 3; ++r) timed(c, "grad32", [&] { launch_grad(c->d_model, a, blocks, true, c->stream); });
+                const double g = mean_time(c, "grad32");
+                if (g < best_g) { best_g = g; tu.grad_atoms = per; }
             }
         } catch (...) {
             tu = keep;

@@ -252,3 +252,41 @@ def test_loss_gradient_wide_network(precision, tmp_path):
     else:
         assert lrel.max() <= 1e-4
         assert rel <= 2e-3
+
+
+@pytest.mark.parametrize("per_block", [1, 5, 16, 32])
+@pytest.mark.parametrize("precision", [n2p2_amd.PLAIN_FP64, n2p2_amd.MIXED])
+def test_gradient_tiles(models, precision, per_block):
+    """The gradient kernel's tiles of atoms: 352 uneven structures (15 to 48
+    atoms, so a tile of 16 holds parts of several and its last one is partly
+    filled) as 32 copies of 11, against the rows of the 11 alone (tiles of a
+    few atoms, pinned to the oracle above).  The terms are equal and only the
+    order of the FP64 sums differs: 1e-12 relative covers their 352 x 48
+    terms.  The summed gradient's residuals come from FP64 forces that differ
+    in the last place, which in the mixed form can round an FP32 seed the
+    other way: 6e-8 of a few of 11,000 atoms' terms, below 1e-9 of the sum."""
+    say("case: gradient tiles, 352 structures, %d atoms per block, precision %d" % (per_block, precision))
+    student, _ = models
+    parts = [synth.water_set(1, m, m, seed=synth.SEED_WATERSET + m) for m in range(5, 16)]
+    pos, elem, boxes = (np.concatenate([p[k] for p in parts]) for k in range(3))
+    off = np.concatenate([[0], np.cumsum([len(p[1]) for p in parts])])
+    rng = np.random.default_rng(51)
+    vE, vF = rng.normal(size=11), rng.normal(size=(len(elem), 3))
+    m = n2p2_amd.Mode(student)
+    m.set_structures(pos, elem, boxes, off)
+    few = m.weight_vjp(vE, vF, precision)
+    E0, F0 = m.energies(), m.forces()
+    _, g0 = m.loss_gradient(E0 - vE, F0 - vF, BETA, precision)
+    n = 32  # a power of two: the scaled weight of the force term is exact
+    t = m.tuning()
+    m.set_tuning(t["trip_sf"], t["trip_force"], t["trip_tangent"], per_block)
+    m.set_structures(np.tile(pos, (n, 1)), np.tile(elem, n), np.tile(boxes, (n, 1, 1)),
+                     np.concatenate([[0], np.cumsum(np.tile(np.diff(off), n))]))
+    rows = m.weight_vjp(np.tile(vE, n), np.tile(vF, (n, 1)), precision)
+    ref = np.tile(few, (n, 1))
+    rel = float(np.abs(rows - ref).max() / np.abs(ref).max())
+    _, g = m.loss_gradient(np.tile(E0 - vE, n), np.tile(F0 - vF, (n, 1)), BETA * n, precision)
+    relg = float(np.abs(g - n * g0).max() / np.abs(n * g0).max())
+    say("  rows max rel %.2e, summed gradient max rel %.2e" % (rel, relg))
+    assert rel <= 1e-12
+    assert relg <= (1e-12 if precision == n2p2_amd.PLAIN_FP64 else 1e-9)
