@@ -91,6 +91,10 @@ void launch_sfcomp32(const ModelT* m, const ModelT& hm, const SysView& s, double
 void launch_tangentcomp32(const ModelT* m, const ModelT& hm, const SysView& s, const double* u, double* Gdot,
                           int ldG, hipStream_t stream);
 
+// ... with FP64 terms.
+void launch_tangentcomp64(const ModelT* m, const ModelT& hm, const SysView& s, const double* u, double* Gdot,
+                          int ldG, hipStream_t stream);
+
 // FP64 atomic NNs over per-element atom lists; dE/dG by the adjoint.
 struct NNIO {
     const double* G;       // [N*ldG] scaled SFs
@@ -132,7 +136,11 @@ void launch_sfcomp64_force(const ModelT* m, const ModelT& hm, const SysView& s, 
 // fused kernels' staging and compacted triplet walk.
 void launch_values64(const ModelT* m, const ModelT& hm, const MixedModel& mm, const SysView& s, double* G, int ldG,
                      hipStream_t stream);
-// LDS bytes of the fused FP64 force kernel at a list capacity (<= 65536 to run).
+// Tangent Gdot = sum_a dG/dx_a . u_a of every SF (Gaussian and compact) in
+// FP64, recomputed as the forces are; fac as in launch_force64_fused.
+void launch_tangent64_fused(const ModelT* m, const ModelT& hm, const MixedModel& mm, const SysView& s,
+                            const double* u, const double* fac, double* Gdot, int ldG, hipStream_t stream);
+// LDS bytes of the fused FP64 kernels at a list capacity (<= 65536 to run).
 size_t fused64_lds(int cap);
 
 // Extrapolation warnings (Element::updateSymmetryFunctionStatistics): every

@@ -105,6 +105,9 @@ struct nnpx_ctx {
     bool rev_valid = false;
     // results state
     bool sf_valid = false, sfd_valid = false, nn_valid = false, dedg_valid = false;
+    // the plain gradient calls leave dG/dr to be had like the results: it is
+    // stored when a call asks for it (stored_dgdr)
+    bool dgdr_due = false;
     bool e_valid = false, f_valid = false;
     int last_precision = NNPX_PLAIN_FP64;
     bool last_stored = false;    // the last plain evaluation stored dG/dr
@@ -334,6 +337,7 @@ void need_structures(nnpx_ctx* c)
 void invalidate(nnpx_ctx* c)
 {
     c->sf_valid = c->sfd_valid = c->nn_valid = c->dedg_valid = c->e_valid = c->f_valid = false;
+    c->dgdr_due = false;
 }
 
 double list_cutoff(const nnpx_ctx* c) { return c->hm.t.maxCutoff + c->skin; }
@@ -577,6 +581,16 @@ void compute_nn64(nnpx_ctx* c, bool deriv)
     });
     c->nn_valid = true;
     c->dedg_valid = deriv;
+}
+
+// Whether dG/dr is stored, storing it first where a gradient call left it due.
+bool stored_dgdr(nnpx_ctx* c)
+{
+    if (!c->sfd_valid && c->dgdr_due) {
+        compute_sf64(c, true);
+        c->dgdr_due = false;
+    }
+    return c->sfd_valid;
 }
 
 // Plain-form forces without stored dG/dr (the fused FP64 kernel); needs the
@@ -1222,7 +1236,7 @@ nnpx_status nnpx_calculate_symmetry_function_groups(nnpx_ctx* c, int derivatives
         need_structures(c);
         if (!c->nbr_valid) build_neighbors(c, true);
         // Mode.cpp:1634-1635: skip when results are already there
-        if (c->sfd_valid || (c->sf_valid && !derivatives)) return;
+        if (stored_dgdr(c) || (c->sf_valid && !derivatives)) return;
         compute_sf64(c, derivatives != 0);
         c->nn_valid = c->dedg_valid = c->e_valid = c->f_valid = false;
     });
@@ -1251,7 +1265,7 @@ nnpx_status nnpx_calculate_forces(nnpx_ctx* c)
 {
     return guard(c, [&] {
         need_structures(c);
-        if (!c->sfd_valid) fail(NNPX_ERR_STATE, "symmetry function derivatives not calculated");
+        if (!stored_dgdr(c)) fail(NNPX_ERR_STATE, "symmetry function derivatives not calculated");
         if (!c->dedg_valid) fail(NNPX_ERR_STATE, "dE/dG not calculated");
         compute_force64(c);
     });
@@ -1364,7 +1378,7 @@ nnpx_status nnpx_get_dGdr(nnpx_ctx* c, double* self, int ld_self, double* nbr, i
 {
     return guard(c, [&] {
         need_structures(c);
-        if (!c->sfd_valid || c->last_precision != NNPX_PLAIN_FP64)
+        if (!stored_dgdr(c) || c->last_precision != NNPX_PLAIN_FP64)
             fail(NNPX_ERR_STATE, "stored dG/dr not available (plain form with derivatives required)");
         settle(c);
         const ModelT& t = c->hm.t;
@@ -1615,7 +1629,12 @@ void weight_vjp(nnpx_ctx* c, int precision, const double* u, const double* cE, d
     double* Gdot = buf<double>(c, "t_Gdot", (size_t)N * ldG);
     hip_check(hipMemsetAsync(Gdot, 0, sizeof(double) * (size_t)N * ldG, c->stream), "hipMemsetAsync");
     SysView s = sysview(c);
-    if (precision == NNPX_PLAIN_FP64) {
+    if (precision == NNPX_PLAIN_FP64 && !c->last_stored) {
+        timed(c, "tangent64f", [&] {
+            launch_tangent64_fused(c->d_model, t, c->mixed, s, u, model_table<double>(c, "fac64"), Gdot, ldG,
+                                   c->stream);
+        });
+    } else if (precision == NNPX_PLAIN_FP64) {
         timed(c, "tangent64", [&] {
             launch_tangent64(c->d_model, s, existing<double>(c, "dGself"), existing<double>(c, "dGnbr"),
                              std::max(t.max_sfd, 1), model_table<int>(c, "islot"), u, Gdot, ldG, c->stream);
@@ -1638,6 +1657,27 @@ void weight_vjp(nnpx_ctx* c, int precision, const double* u, const double* cE, d
     if (ldgrad == 0) a.part = buf<double>(c, "t_part", (size_t)blocks * a.nconn_max);
     timed(c, precision == NNPX_MIXED ? "grad32" : "grad64",
           [&] { launch_grad(c->d_model, a, blocks, precision == NNPX_MIXED, c->stream); });
+}
+
+// The evaluation before a gradient: forces, and for the plain form the state
+// the tangent needs.  During MD the plain form stores dG/dr (the fused kernels'
+// staging is fitted to the MD run, not to this list).
+void gradient_evaluate(nnpx_ctx* c, int precision)
+{
+    const bool plain = precision == NNPX_PLAIN_FP64;
+    evaluate(c, precision, NNPX_EVAL_FORCES, true, plain && c->md_ready);
+    settle(c);
+    c->dgdr_due = plain && !c->last_stored;
+}
+
+// Forces seeds [3 * force entries] of the gradient calls; entries past the
+// evaluated atoms (ghosts of an external list) are zero.
+double* seed_buffer(nnpx_ctx* c)
+{
+    const size_t n = (size_t)3 * force_entries(c);
+    double* u = buf<double>(c, "t_u", n);
+    if (c->external) hip_check(hipMemsetAsync(u, 0, sizeof(double) * n, c->stream), "hipMemsetAsync");
+    return u;
 }
 
 int total_connections(const ModelT& t)
@@ -1665,15 +1705,14 @@ nnpx_status nnpx_loss_gradient(nnpx_ctx* c, int precision, const double* E_ref, 
         gradient_checks(c, precision);
         if (!E_ref || !F_ref || !loss || !grad) fail(NNPX_ERR_ARGUMENT, "null argument");
         if (!(beta >= 0.0)) fail(NNPX_ERR_ARGUMENT, "beta must be >= 0");
-        evaluate(c, precision, NNPX_EVAL_FORCES, true, precision == NNPX_PLAIN_FP64);
-        settle(c);
+        gradient_evaluate(c, precision);
         const int N = c->N, S = c->S;
         double* Eref = buf<double>(c, "t_Eref", S);
         double* Fref = buf<double>(c, "t_Fref", (size_t)3 * N);
         hip_check(hipMemcpyAsync(Eref, E_ref, sizeof(double) * S, hipMemcpyHostToDevice, c->stream), "hipMemcpyAsync");
         hip_check(hipMemcpyAsync(Fref, F_ref, sizeof(double) * 3 * N, hipMemcpyHostToDevice, c->stream),
                   "hipMemcpyAsync");
-        double* u = buf<double>(c, "t_u", (size_t)3 * N);
+        double* u = seed_buffer(c);
         double* cE = buf<double>(c, "t_cE", S);
         double* lossd = buf<double>(c, "t_loss", 4);
         const int total = total_connections(c->hm.t);
@@ -1700,11 +1739,10 @@ nnpx_status nnpx_weight_vjp(nnpx_ctx* c, int precision, const double* vE, const 
     return guard(c, [&] {
         gradient_checks(c, precision);
         if (!vE || !vF || !grad) fail(NNPX_ERR_ARGUMENT, "null argument");
-        evaluate(c, precision, NNPX_EVAL_FORCES, true, precision == NNPX_PLAIN_FP64);
-        settle(c);
+        gradient_evaluate(c, precision);
         const int N = c->N, S = c->S;
         const int total = total_connections(c->hm.t);
-        double* u = buf<double>(c, "t_u", (size_t)3 * N);
+        double* u = seed_buffer(c);
         double* cE = buf<double>(c, "t_cE", S);
         double* gd = buf<double>(c, "t_gradS", (size_t)S * total);
         hip_check(hipMemcpyAsync(cE, vE, sizeof(double) * S, hipMemcpyHostToDevice, c->stream), "hipMemcpyAsync");
@@ -1805,8 +1843,7 @@ nnpx_status nnpx_kalman_update(nnpx_ctx* c, int precision, int property, int bat
         const bool force = property == 1;
         const double fw = force ? force_weight : 1.0;
         // Errors of the current weights (Training::update PART 2)
-        evaluate(c, precision, NNPX_EVAL_FORCES, true, precision == NNPX_PLAIN_FP64);
-        settle(c);
+        gradient_evaluate(c, precision);
         std::vector<double> E(S), F((size_t)3 * N);
         copy_out(c, E.data(), existing<double>(c, "E"), sizeof(double) * S);
         if (force) copy_out(c, F.data(), existing<double>(c, "F"), sizeof(double) * 3 * N);
@@ -1848,7 +1885,7 @@ nnpx_status nnpx_kalman_update(nnpx_ctx* c, int precision, int property, int bat
         // summed row, or one row per candidate in rounds of candidates on
         // different structures
         std::vector<double> rows((size_t)m * total, 0.0);
-        double* u = buf<double>(c, "t_u", (size_t)3 * N);
+        double* u = seed_buffer(c);
         double* cE = buf<double>(c, "t_cE", S);
         double* gd = buf<double>(c, "t_gradS", (size_t)S * total);
         std::vector<int> done(batch, 0);
@@ -1984,7 +2021,7 @@ nnpx_status nnpx_autotune(nnpx_ctx* c)
         double best_t = 1e30;
         Tuning best = keep;
         const int ldG = t.max_sf;
-        double* u = buf<double>(c, "t_u", (size_t)3 * c->N);
+        double* u = seed_buffer(c);
         double* Gdot = buf<double>(c, "t_Gdot", (size_t)c->N * ldG);
         hip_check(hipMemsetAsync(u, 0, sizeof(double) * 3 * c->N, c->stream), "hipMemsetAsync");
         try {

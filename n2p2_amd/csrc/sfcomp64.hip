@@ -584,6 +584,20 @@ void launch_tangentcomp32(const ModelT* m, const ModelT& hm, const SysView& s, c
                        capL);
 }
 
+void launch_tangentcomp64(const ModelT* m, const ModelT& hm, const SysView& s, const double* u, double* Gdot,
+                          int ldG, hipStream_t stream)
+{
+    if (s.natoms == 0 || !hm.has_comp) return;
+    const int capL = ((std::max(s.cap, 1) + 31) / 32) * 32;
+    const size_t lds = comp_lds(capL, 1);
+    if (lds > 65536)
+        throw Error{NNPX_ERR_UNSUPPORTED, "neighbour count too large for the FP64 compact SF kernel's LDS staging"};
+    const SF64Out o{};
+    const CompMix c{Gdot, nullptr, ldG, 0, nullptr, nullptr, 0, u};
+    hipLaunchKernelGGL((k_sfcomp<double, CM_TANGENT, 16>), dim3(s.natoms), dim3(kCThreads), lds, stream, m, s, o, c, 0,
+                       capL);
+}
+
 void launch_sfcomp32(const ModelT* m, const ModelT& hm, const SysView& s, double* G, float* Gin, int ldG, int ldK,
                      const float* fw, double* F, bool push, bool forces, hipStream_t stream)
 {
