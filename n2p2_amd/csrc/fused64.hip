@@ -46,6 +46,7 @@
 #include "kernels.hpp"
 #include "mixed.hpp"
 #include "nnpx.h"
+#include "stage.hpp"
 
 namespace nnpx {
 namespace {
@@ -54,7 +55,6 @@ namespace {
 // values 355 us at 256 pairs, 377 at 384; forces 553, 551).
 constexpr int kWalk64 = 256;
 constexpr int kMinWalk64 = 128;  // ... at least
-constexpr int kPasses64 = 16;    // 64-entry passes of the longest list (1,024 entries)
 constexpr size_t kLds64 = 65536;
 // Atoms up to which four waves share one, else two: 4,096 atoms give every SIMD
 // eight waves of two per atom.  1,300 atoms: four waves 88 + 128 us (values,
@@ -69,7 +69,7 @@ struct Stage64 {
     double* ay;
     double* az;
     unsigned* tjk;       // this wave's compacted pairs (j | k << 16)
-    int* cnt;            // [kPasses64][kMaxElem] staging counts (before the walks, in the waves' pair buffers)
+    int* cnt;            // [kStagePasses][kMaxElem] staging counts (before the walks, in the waves' pair buffers)
     unsigned short* la;  // group lists
     unsigned short* lb;
     unsigned char* el;   // neighbour element
@@ -102,10 +102,6 @@ __host__ __device__ constexpr size_t stage64_bytes(int capL, int waves, int walk
            (size_t)waves * (walk + kWave) * 4 + 48;
 }
 
-// Lane of the wave, and the wave's number in the block as a scalar.
-__device__ inline int lane64() { return threadIdx.x & (kWave - 1); }
-__device__ inline int wave64() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
-
 // Orders a wave's LDS writes before its own later reads (the hardware keeps a
 // wave's LDS accesses in order; this keeps the compiler from moving them).
 __device__ inline void wave_fence()
@@ -127,7 +123,7 @@ __device__ inline Stage64 carve64(double4* base, int capL, int walk)
     S.az = S.ay + capL;
     unsigned* t = reinterpret_cast<unsigned*>(S.az + capL);
     S.cnt = reinterpret_cast<int*>(t);
-    S.tjk = t + wave64() * (walk + kWave);
+    S.tjk = t + wave_id() * (walk + kWave);
     S.la = reinterpret_cast<unsigned short*>(t + W * (walk + kWave));
     S.lb = S.la + capL;
     S.el = reinterpret_cast<unsigned char*>(S.lb + capL);
@@ -136,103 +132,24 @@ __device__ inline Stage64 carve64(double4* base, int capL, int walk)
     return S;
 }
 
-// Stages the atom's list entries closer than the model's largest cutoff
-// (entries beyond it contribute nothing; MD lists built with a skin carry
-// them), grouped by neighbour element and in list order within an element,
-// so element e's neighbours are the slots eoff[e] .. eoff[e + 1] - 1; each
+// Stages the atom's in-cutoff list entries (stage_by_element): geometry, each
 // slot's list entry in idx and, for the force kernel, zeroed neighbour force
-// sums.  Wave w takes the list's 64-entry passes w, w + W, ...  More such
-// entries than capL: only slots below capL are staged, flag bit 4 is set (the
-// caller repeats with the full capacity) and flags[2] keeps the largest count
-// met.
+// sums.
 template <int W>
 __device__ inline int stage64(const ModelT* __restrict__ M, const SysView& s, int i, int capL, const Stage64& S,
                               bool zero_sums)
 {
-    const int lane = lane64(), wv = wave64();
-    const StructT& St = s.st[s.sid[i]];
-    const int nl = s.nb_n[i];
-    const int ne = M->nelem;
-    const int npass = min((nl + kWave - 1) / kWave, kPasses64);
-    const size_t base = (size_t)i * s.cap;
-    const double rmax = M->maxCutoff;
-    struct Entry {
-        double dr[3], d;
-        int el;
-    };
-    auto entry = [&](int p) {
-        Entry x{{0.0, 0.0, 0.0}, 0.0, -1};
-        const int k = p * kWave + lane;
-        if (k < nl) {
-            entry_vector(s, i, base + k, St, x.dr);
-            x.d = sqrt(x.dr[0] * x.dr[0] + x.dr[1] * x.dr[1] + x.dr[2] * x.dr[2]);
-            if (x.d < rmax) x.el = s.elem[s.nb_j[base + k]];
+    return stage_by_element<W>(M, s, i, capL, S.cnt, S.eoff, [&](int pos, int k, const double* dr, double d, int el) {
+        S.g[pos] = make_double4(dr[0], dr[1], dr[2], d);
+        S.c[pos] = make_double4(1.0 / d, 0.0, 0.0, M->Zel[el]);
+        S.el[pos] = (unsigned char)el;
+        S.idx[pos] = (unsigned short)k;
+        if (zero_sums) {
+            S.ax[pos] = 0.0;
+            S.ay[pos] = 0.0;
+            S.az[pos] = 0.0;
         }
-        return x;
-    };
-    // in-cutoff entries per pass and element; a wave's first passes stay in
-    // registers for the placing (lists up to kKeep * W * 64 entries)
-    constexpr int kKeep = W >= 4 ? 1 : 4 / W;
-    Entry keep[kKeep];
-    auto count = [&](int p, int el) {
-        for (int e = 0; e < ne; ++e) {
-            const int c = __popcll(__ballot(el == e));
-            if (lane == 0) S.cnt[p * kMaxElem + e] = c;
-        }
-    };
-#pragma unroll
-    for (int q = 0; q < kKeep; ++q) {
-        const int p = wv + q * W;
-        keep[q].el = -1;
-        if (p < npass) {
-            keep[q] = entry(p);
-            count(p, keep[q].el);
-        }
-    }
-    for (int p = wv + kKeep * W; p < npass; p += W) count(p, entry(p).el);
-    __syncthreads();
-    // lane e: element e's entries, its first slot, and the next of this wave's pass
-    int tot = 0;
-    if (lane < ne)
-        for (int p = 0; p < npass; ++p) tot += S.cnt[p * kMaxElem + lane];
-    const int incl = wave_incl_scan(tot);
-    const int total = lane_value(incl, kWave - 1);
-    int next = incl - tot, seen = 0;
-    if (wv == 0 && lane <= ne) S.eoff[lane] = min(lane < ne ? next : total, capL);
-    auto place = [&](int p, const Entry& x) {
-        for (; seen < p; ++seen)
-            if (lane < ne) next += S.cnt[seen * kMaxElem + lane];
-        int pos = -1;
-        for (int e = 0; e < ne; ++e) {
-            const unsigned long long m = __ballot(x.el == e);
-            const int at = lane_value(next, e);
-            if (x.el == e)
-                pos = at + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                          __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-        }
-        if (pos >= 0 && pos < capL) {
-            S.g[pos] = make_double4(x.dr[0], x.dr[1], x.dr[2], x.d);
-            S.c[pos] = make_double4(1.0 / x.d, 0.0, 0.0, M->Zel[x.el]);
-            S.el[pos] = (unsigned char)x.el;
-            S.idx[pos] = (unsigned short)(p * kWave + lane);
-            if (zero_sums) {
-                S.ax[pos] = 0.0;
-                S.ay[pos] = 0.0;
-                S.az[pos] = 0.0;
-            }
-        }
-    };
-#pragma unroll
-    for (int q = 0; q < kKeep; ++q)
-        if (wv + q * W < npass) place(wv + q * W, keep[q]);
-    for (int p = wv + kKeep * W; p < npass; p += W) place(p, entry(p));
-    if (threadIdx.x == 0) {
-        if (total > capL) atomicOr(&s.flags[0], 4);
-        if (total > __hip_atomic_load(&s.flags[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            atomicMax(&s.flags[2], total);
-    }
-    __syncthreads();
-    return __builtin_amdgcn_readfirstlane(min(total, capL));
+    });
 }
 
 // sqrt(x) and 1/sqrt(x): the hardware's reciprocal square root (about 2^-28)
@@ -360,7 +277,7 @@ template <int W>
 __device__ inline List64 make_list64(const ModelT* __restrict__ M, const Stage64& S, int n, const GroupT& G, int elem,
                                      unsigned short* out)
 {
-    const int lane = lane64();
+    const int lane = lane_id();
     const int lo = __builtin_amdgcn_readfirstlane(elem < 0 ? 0 : S.eoff[elem]);
     const int hi = __builtin_amdgcn_readfirstlane(elem < 0 ? n : S.eoff[elem + 1]);
     List64 L{lo, hi - lo, true};
@@ -369,7 +286,7 @@ __device__ inline List64 make_list64(const ModelT* __restrict__ M, const Stage64
         for (int b = lo; b < hi; b += kWave) {
             const int k = b + lane;
             const unsigned long long m = __ballot(k < hi && S.g[k].w < G.rc);
-            if (wave64() == 0 && (m >> lane) & 1)
+            if (wave_id() == 0 && (m >> lane) & 1)
                 out[cnt + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                          __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
                     (unsigned short)k;
@@ -393,7 +310,7 @@ template <int W, bool CONTIG, typename Work, typename Flush>
 __device__ inline void triplets64(const Stage64& S, const List64& A, const List64& B, bool same, double rc2,
                                  Work&& work, Flush&& flush)
 {
-    const int lane = lane64();
+    const int lane = lane_id();
     const int nA = A.n, nB = B.n;
     const int R = same ? (nA - 1) / 2 : nB;          // regular columns per row
     const int Rx = same && nA % 2 == 0 ? R + 1 : R;  // with the half-way column (rows a < nA / 2 only)
@@ -405,7 +322,7 @@ __device__ inline void triplets64(const Stage64& S, const List64& A, const List6
     const bool live = lr < rh;
     const unsigned short* lb = same ? S.la : S.lb;
     const int bB = same ? A.base : B.base;
-    int a0 = wave64() * rh, c0 = 0;
+    int a0 = wave_id() * rh, c0 = 0;
     int ja = 0;
     double gx = 0.0, gy = 0.0, gz = 0.0;
     auto row = [&] {
@@ -538,7 +455,7 @@ __global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(4, 4)
     extern __shared__ double4 sm64[];
     const Stage64 S = carve64<W>(sm64, capL, walk);
     const int i = blockIdx.x;
-    const int lane = lane64();
+    const int lane = lane_id();
     const int e = s.elem[i];
     const ElementT& E = M->el[e];
     const int ctype = M->cutoffType;
@@ -718,7 +635,7 @@ __global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(4, 4)
     fy = wave_sum(fy);
     fz = wave_sum(fz);
     if (lane == 0) {
-        double* r = S.red + wave64() * 3;
+        double* r = S.red + wave_id() * 3;
         r[0] = fx;
         r[1] = fy;
         r[2] = fz;
@@ -765,7 +682,7 @@ __global__ __launch_bounds__(kWave * W) void k_values64(const ModelT* __restrict
     extern __shared__ double4 sm64[];
     const Stage64 S = carve64<W>(sm64, capL, walk);
     const int i = blockIdx.x;
-    const int lane = lane64(), wv = wave64();
+    const int lane = lane_id(), wv = wave_id();
     const int e = s.elem[i];
     const ElementT& E = M->el[e];
     const int ctype = M->cutoffType;

@@ -26,6 +26,7 @@
 
 #include "mixed.hpp"
 #include "nnpx.h"
+#include "sfcomp.hpp"
 
 namespace nnpx {
 namespace {
@@ -2483,8 +2484,11 @@ void run_mixed(const MixedModel& mm, const ModelT& t, const ModelT* d_model, con
     T.rows = !lists;
     // the staging passes from the SF to the force kernel (identical values)
     const StageKeep KS = forces && b.keep.ld >= capL ? b.keep : StageKeep{};
+    // a model of compact functions alone leaves these kernels nothing: its
+    // values (and the input rows' padding) come from the factored kernel
+    const bool gauss_sf = t.has_exp || !sfcomp_factored_fits<float>(CM_VALUES, capL);
     timed("sf32", [&] {
-        dispatch_angular(mm, P, [&](auto m, auto fast, auto nb0, auto nb1) {
+        if (gauss_sf) dispatch_angular(mm, P, [&](auto m, auto fast, auto nb0, auto nb1) {
             constexpr int cm = decltype(m)::value, c0 = decltype(nb0)::value, c1 = decltype(nb1)::value;
             constexpr bool cf = decltype(fast)::value;
             constexpr bool cmg = c0 > 0;  // merged instances exist on the power path only
@@ -2563,7 +2567,7 @@ void run_mixed(const MixedModel& mm, const ModelT& t, const ModelT* d_model, con
             hipLaunchKernelGGL(k_zero, dim3((unsigned)std::min<size_t>((n3 + 255) / 256, 4096)), dim3(256), 0,
                                stream, b.F, n3);
         const int ps = push ? 1 : 0;
-        dispatch_angular(mm, P, [&](auto m, auto fast, auto nb0, auto nb1) {
+        if (t.has_exp) dispatch_angular(mm, P, [&](auto m, auto fast, auto nb0, auto nb1) {
             constexpr int cm = decltype(m)::value, c0 = decltype(nb0)::value, c1 = decltype(nb1)::value;
             constexpr bool cf = decltype(fast)::value;
             const bool mg = c0 > 0 && merge_f;

@@ -179,6 +179,40 @@ void compact_subtype(SF& f)
     }
 }
 
+// The factored form of compact group G (CompFactorT), where it is wide, has
+// at most kCompU radial and kCompV angular functions and no member twice.
+void factor_group(ModelT& t, GroupT& G)
+{
+    G.fac = 0;
+    if (!sf_compact(G.type) || sf_radial(G.type)) return;
+    auto index = [](CompWindowT* w, int& n, int most, const CompWindowT& x) {
+        for (int k = 0; k < n; ++k)
+            if (w[k].core == x.core && w[k].asym == x.asym && w[k].lo == x.lo && w[k].hi == x.hi) return k;
+        if (n == most) return -1;
+        w[n] = x;
+        return n++;
+    };
+    CompFactorT f{};
+    std::fill(f.cell, f.cell + kCompU * kCompV, (signed char)-1);
+    bool ok = (G.type == 22 || G.type == 25) && t.nfactored < kMaxFactored;
+    for (int q = 0; q < G.nmem && ok; ++q) {
+        const MemberT& M = t.mem[G.mem0 + q];
+        const int u = index(f.rad, f.U, kCompU, CompWindowT{M.core, M.asym, M.rl, M.rcm, M.cen, M.scl});
+        const int v = index(f.ang, f.V, kCompV, CompWindowT{M.core, 0, M.al, M.ar, M.acen, M.ascl});
+        ok = u >= 0 && v >= 0 && f.cell[u * kCompV + v] < 0;
+        if (ok) f.cell[u * kCompV + v] = (signed char)q;
+    }
+    if (!ok) {
+        t.has_unfactored = 1;
+        return;
+    }
+    if (t.nfactored == 0) t.fac_poly2 = 1;
+    for (int q = 0; q < G.nmem; ++q)
+        if (t.mem[G.mem0 + q].core != 2) t.fac_poly2 = 0;
+    t.cfac[t.nfactored] = f;
+    G.fac = ++t.nfactored;
+}
+
 }  // namespace
 
 void load_model(const std::string& dir, HostModel& hm)
@@ -482,6 +516,7 @@ void load_model(const std::string& dir, HostModel& hm)
                 }
             }
         }
+        for (int g = E.grp0; g < gcount; ++g) factor_group(t, t.grp[g]);
         sfcount += E.nsf;
         t.max_sf = std::max(t.max_sf, E.nsf);
     }

@@ -40,7 +40,7 @@ struct GroupT {
     int e1, e2;      // neighbour elements (e1 <= e2)
     int nmem;        // members
     int mem0;        // first member in ModelT::mem
-    int pad;
+    int fac;         // compact wide: 1 + index in ModelT::cfac, 0: not factored
     double rc, rc2;
     double rcinv, rci, iw;  // cutoff constants (CutoffFunction.cpp:95-112)
     double rmin;     // compact: lower radial bound of the group
@@ -72,6 +72,22 @@ struct MemberT {
     double cen, scl;     // radial centre and 1/half-width
     double al, ar;       // angular window (radians)
     double acen, ascl;   // angular centre and 1/half-width
+};
+
+// A wide compact group (types 22, 25) as the product of its distinct radial
+// and angular functions: every member is radial function u at both neighbours
+// times angular function v, cell[u * kCompV + v] its index in the group (-1:
+// the group has no such member).
+constexpr int kCompU = 9, kCompV = 6;
+constexpr int kMaxFactored = 256;
+struct CompWindowT {
+    int core, asym;  // as in MemberT
+    double lo, hi, cen, scl;
+};
+struct CompFactorT {
+    int U, V;
+    CompWindowT rad[kCompU], ang[kCompV];
+    signed char cell[kCompU * kCompV];
 };
 
 // SymFnc::scale (SymFnc.cpp:169-195): Smin + factor * (v - shift) or v - shift.
@@ -115,6 +131,9 @@ struct ModelT {
     int max_mem_comp;       // max members of a compact angular group
     int has_exp;            // any Gaussian (type 2/3/9) group
     int has_comp;           // any compact (type 20-25) group
+    int has_unfactored;     // any compact angular group without a factored form
+    int nfactored;          // entries of cfac
+    int fac_poly2;          // every core in them is the second polynomial
     int has_weighted;       // any element-weighted (type 12/13/23/24/25) group
     double Zel[kMaxElem];   // atomic number by element index
     int max_width;          // max NN layer width (input layer included)
@@ -125,6 +144,7 @@ struct ModelT {
     double tanhPre;         // CT_TANH prefactor (CutoffFunction.cpp:28)
     ElementT el[kMaxElem];
     GroupT grp[kMaxElem * kMaxGroups];
+    CompFactorT cfac[kMaxFactored];
     MemberT mem[kMaxElem * kMaxSF];
     ScaleT scale[kMaxElem * kMaxSF];
     int table[kMaxElem * kMaxElem * kMaxSF];  // slot -> SF index

@@ -18,6 +18,10 @@
 //    u, the mixed training gradient's tangent (Training::collectDGdxia
 //    contracted with u, Training.cpp:3586-3625).
 //
+// Radial groups and the angular groups that have a factored form
+// (CompFactorT) are left to the factored kernel (sfcomp_fac.hip) where `skip`
+// is set.
+//
 // Mapping: one 256-thread workgroup per atom with the neighbour geometry
 // staged in LDS.  Radial groups: threads over neighbours, members in
 // sequence.  Angular groups: threads over the unordered neighbour pairs of
@@ -28,8 +32,8 @@
 // windows), so a chunk keeps the accumulators bounded whatever the group size.
 #include <type_traits>
 
-#include "kernels.hpp"
 #include "nnpx.h"
+#include "sfcomp.hpp"
 
 namespace nnpx {
 namespace {
@@ -85,8 +89,6 @@ __device__ inline int build_list(const CLds& L, int n, int elem, double rmin, do
     return c;
 }
 
-enum CompMode { CM_PLAIN = 0, CM_VALUES = 1, CM_FORCE = 2, CM_TANGENT = 3 };
-
 // Member windows and centres in the term precision.
 template <typename T>
 __device__ inline void radial_fdf(const MemberT& m, T r, T& f, T& df)
@@ -113,21 +115,9 @@ __device__ inline bool member_skipped(const MemberT& m, T radij, T rik, T rjk, b
            th <= (T)m.al || th >= (T)m.ar;
 }
 
-// Outputs of the mixed modes.
-struct CompMix {
-    double* G;        // [N*ldG] scaled values (values mode)
-    float* Gin;       // [N*ldK] their FP32 copy, the network input
-    int ldG, ldK;
-    const float* fw;  // [N*ldG] dE/dG times the scaling factor (force mode)
-    double* F;        // forces (force mode)
-    int push;         // keep contributions to the atom's own images
-    const double* u;  // [3N] field of the tangent mode (its output goes to G)
-    const double* fw64;  // [N*ldG] FP64 weights of the FP64 force mode (plain form)
-};
-
 template <typename T, int MODE, int CH>
 __global__ __launch_bounds__(kCThreads) void k_sfcomp(const ModelT* __restrict__ M, SysView s, SF64Out o,
-                                                       CompMix c, int deriv, int capL)
+                                                       CompMix c, int deriv, int capL, int skip)
 {
     constexpr bool PLAIN = MODE == CM_PLAIN, FORCE = MODE == CM_FORCE, TANGENT = MODE == CM_TANGENT;
     constexpr bool DER = PLAIN || TANGENT;  // derivatives times the scaling factor
@@ -198,7 +188,7 @@ __global__ __launch_bounds__(kCThreads) void k_sfcomp(const ModelT* __restrict__
     // ---------------------------------------------------------- radial groups
     for (int gi = 0; gi < E.nrad; ++gi) {
         const GroupT& G = M->grp[E.grp0 + gi];
-        if (G.type != 20 && G.type != 23) continue;
+        if ((G.type != 20 && G.type != 23) || skip) continue;
         // weighted (SymGrpCompRadWeighted.cpp:120-200): every neighbour
         // element, each term times its atomic number
         const bool wt = G.type == 23;
@@ -276,7 +266,7 @@ __global__ __launch_bounds__(kCThreads) void k_sfcomp(const ModelT* __restrict__
     // --------------------------------------------------------- angular groups
     for (int gi = E.nrad; gi < E.ngrp; ++gi) {
         const GroupT& G = M->grp[E.grp0 + gi];
-        if (G.type < 21 || G.type == 23) continue;
+        if (G.type < 21 || G.type == 23 || (skip && G.fac)) continue;
         const bool narrow = G.type == 21 || G.type == 24;
         // weighted (types 24, 25; SymGrpCompAng{n,w}Weighted.cpp): all
         // neighbour pairs, the angular factor times Z_j Z_k
@@ -543,12 +533,19 @@ void launch_sfcomp64(const ModelT* m, const ModelT& hm, const SysView& s, const 
         throw Error{NNPX_ERR_UNSUPPORTED, "neighbour count too large for the FP64 compact SF kernel's LDS staging"};
     const dim3 grid(s.natoms), block(kCThreads);
     const int d = deriv ? 1 : 0;
-    const CompMix c{};
+    CompMix c{};
+    const int skip = !deriv && sfcomp_factored_fits<double>(CM_VALUES, capL) ? 1 : 0;
+    if (skip) {
+        c.G = o.G;
+        c.ldG = o.ldG;
+        launch_sfcomp_factored<double>(m, hm, s, c, CM_VALUES, capL, stream);
+        if (!hm.has_unfactored) return;
+    }
     switch (ch) {
-    case 8: hipLaunchKernelGGL((k_sfcomp<double, CM_PLAIN, 8>), grid, block, lds, stream, m, s, o, c, d, capL); break;
-    case 4: hipLaunchKernelGGL((k_sfcomp<double, CM_PLAIN, 4>), grid, block, lds, stream, m, s, o, c, d, capL); break;
-    case 2: hipLaunchKernelGGL((k_sfcomp<double, CM_PLAIN, 2>), grid, block, lds, stream, m, s, o, c, d, capL); break;
-    default: hipLaunchKernelGGL((k_sfcomp<double, CM_PLAIN, 1>), grid, block, lds, stream, m, s, o, c, d, capL); break;
+    case 8: hipLaunchKernelGGL((k_sfcomp<double, CM_PLAIN, 8>), grid, block, lds, stream, m, s, o, c, d, capL, skip); break;
+    case 4: hipLaunchKernelGGL((k_sfcomp<double, CM_PLAIN, 4>), grid, block, lds, stream, m, s, o, c, d, capL, skip); break;
+    case 2: hipLaunchKernelGGL((k_sfcomp<double, CM_PLAIN, 2>), grid, block, lds, stream, m, s, o, c, d, capL, skip); break;
+    default: hipLaunchKernelGGL((k_sfcomp<double, CM_PLAIN, 1>), grid, block, lds, stream, m, s, o, c, d, capL, skip); break;
     }
 }
 
@@ -566,8 +563,11 @@ void launch_sfcomp64_force(const ModelT* m, const ModelT& hm, const SysView& s, 
     c.F = F;
     c.push = push ? 1 : 0;
     c.fw64 = w;
+    const int skip = sfcomp_factored_fits<double>(CM_FORCE, capL) ? 1 : 0;
+    if (skip) launch_sfcomp_factored<double>(m, hm, s, c, CM_FORCE, capL, stream);
+    if (skip && !hm.has_unfactored) return;
     hipLaunchKernelGGL((k_sfcomp<double, CM_FORCE, 1>), dim3(s.natoms), dim3(kCThreads), lds, stream, m, s, o, c, 0,
-                       capL);
+                       capL, skip);
 }
 
 void launch_tangentcomp32(const ModelT* m, const ModelT& hm, const SysView& s, const double* u, double* Gdot,
@@ -580,8 +580,11 @@ void launch_tangentcomp32(const ModelT* m, const ModelT& hm, const SysView& s, c
         throw Error{NNPX_ERR_UNSUPPORTED, "neighbour count too large for the mixed compact SF kernel's LDS staging"};
     const SF64Out o{};
     const CompMix c{Gdot, nullptr, ldG, 0, nullptr, nullptr, 0, u};
+    const int skip = sfcomp_factored_fits<float>(CM_TANGENT, capL) ? 1 : 0;
+    if (skip) launch_sfcomp_factored<float>(m, hm, s, c, CM_TANGENT, capL, stream);
+    if (skip && !hm.has_unfactored) return;
     hipLaunchKernelGGL((k_sfcomp<float, CM_TANGENT, 16>), dim3(s.natoms), dim3(kCThreads), lds, stream, m, s, o, c, 0,
-                       capL);
+                       capL, skip);
 }
 
 void launch_tangentcomp64(const ModelT* m, const ModelT& hm, const SysView& s, const double* u, double* Gdot,
@@ -594,8 +597,11 @@ void launch_tangentcomp64(const ModelT* m, const ModelT& hm, const SysView& s, c
         throw Error{NNPX_ERR_UNSUPPORTED, "neighbour count too large for the FP64 compact SF kernel's LDS staging"};
     const SF64Out o{};
     const CompMix c{Gdot, nullptr, ldG, 0, nullptr, nullptr, 0, u};
+    const int skip = sfcomp_factored_fits<double>(CM_TANGENT, capL) ? 1 : 0;
+    if (skip) launch_sfcomp_factored<double>(m, hm, s, c, CM_TANGENT, capL, stream);
+    if (skip && !hm.has_unfactored) return;
     hipLaunchKernelGGL((k_sfcomp<double, CM_TANGENT, 16>), dim3(s.natoms), dim3(kCThreads), lds, stream, m, s, o, c, 0,
-                       capL);
+                       capL, skip);
 }
 
 void launch_sfcomp32(const ModelT* m, const ModelT& hm, const SysView& s, double* G, float* Gin, int ldG, int ldK,
@@ -609,8 +615,12 @@ void launch_sfcomp32(const ModelT* m, const ModelT& hm, const SysView& s, double
     const dim3 grid(s.natoms), block(kCThreads);
     const SF64Out o{};
     const CompMix c{G, Gin, ldG, ldK, fw, F, push ? 1 : 0, nullptr};
-    if (forces) hipLaunchKernelGGL((k_sfcomp<float, CM_FORCE, 1>), grid, block, lds, stream, m, s, o, c, 0, capL);
-    else hipLaunchKernelGGL((k_sfcomp<float, CM_VALUES, 16>), grid, block, lds, stream, m, s, o, c, 0, capL);
+    const CompMode mode = forces ? CM_FORCE : CM_VALUES;
+    const int skip = sfcomp_factored_fits<float>(mode, capL) ? 1 : 0;
+    if (skip) launch_sfcomp_factored<float>(m, hm, s, c, mode, capL, stream);
+    if (skip && !hm.has_unfactored) return;
+    if (forces) hipLaunchKernelGGL((k_sfcomp<float, CM_FORCE, 1>), grid, block, lds, stream, m, s, o, c, 0, capL, skip);
+    else hipLaunchKernelGGL((k_sfcomp<float, CM_VALUES, 16>), grid, block, lds, stream, m, s, o, c, 0, capL, skip);
 }
 
 }  // namespace nnpx
