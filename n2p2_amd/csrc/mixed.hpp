@@ -58,19 +58,19 @@ struct GroupPow64 {
 
 // LDS staging of the mixed kernels: float4 slots of the per-group constant
 // area (member constants, two per member, on the member paths; one per term
-// on the power path) ...
-__host__ __device__ constexpr int stage_mp(int nb0, int nb1)
+// on the power path, where it also takes each wave's FP64 sum per term) ...
+__host__ __device__ constexpr int stage_mp(int nb0, int nb1, int waves)
 {
-    return nb0 > 0 ? 2 * (nb0 + nb1) : 2 * kMaxMembersExp;
+    return nb0 > 0 ? (waves > 2 ? waves : 2) * (nb0 + nb1) : 2 * kMaxMembersExp;
 }
 // ... and bytes of the whole staging area: per slot geometry, cutoffs, two
-// list entries and the element; the triplet buffer (trip entries and up to a
-// wave's worth carried past them); the constants; the element offsets (capL
-// is a multiple of 32 and trip of 64, so the byte arrays end 16-byte
+// list entries and the element; each wave's triplet buffer (trip entries and
+// up to a wave's worth carried past them); the constants; the element offsets
+// (capL is a multiple of 32 and trip of 64, so the byte arrays end 16-byte
 // aligned, as does the offset table)
-__host__ __device__ constexpr size_t stage_bytes(int capL, int trip, int mpn)
+__host__ __device__ constexpr size_t stage_bytes(int capL, int waves, int trip, int mpn)
 {
-    return (size_t)capL * (32 + 2 + 2 + 1) + (size_t)(trip + kWave) * 4 + (size_t)mpn * 16 + 48;
+    return (size_t)capL * (32 + 2 + 2 + 1) + (size_t)waves * (trip + kWave) * 4 + (size_t)mpn * 16 + 48;
 }
 
 // Each atom's compacted angular pairs in device memory, walk by walk (the
@@ -81,9 +81,10 @@ __host__ __device__ constexpr size_t stage_bytes(int capL, int trip, int mpn)
 // the same pairs in the same buffers.  Without lists the force kernel may
 // instead walk rows, whose order suits some models better (the tuning
 // decides).
+constexpr int kListWaves = 4;  // most waves an atom's walks are shared by
 struct TripList {
-    unsigned* list = nullptr;  // [natoms][cap] pairs j | k << 16 (nullptr: none kept)
-    int* counts = nullptr;     // [natoms][ld] pairs of each walk, -1: not kept
+    unsigned* list = nullptr;  // [natoms][cap] pairs j | k << 16 (nullptr: none kept), a share for each wave
+    int* counts = nullptr;     // [natoms][kListWaves][ld] pairs of each wave's walk, -1: not kept
     int cap = 0, ld = 0;
     bool count = false;        // record the largest per-atom pair count in flags[3]
     bool rows = false;         // the force kernel walks rows (no lists kept)
@@ -180,6 +181,12 @@ void setup_mixed(MixedModel& mm, const HostModel& hm);
 void free_mixed(MixedModel& mm);
 void run_mixed(const MixedModel& mm, const ModelT& t, const ModelT* d_model, const SysView& s,
                const MixedBuffers& b, bool forces, bool push, hipStream_t stream, const TimedFn& timed);
+// The kernels of run_mixed (one launch each).
+void launch_sf32(const MixedModel& mm, const ModelT& t, const ModelT* d_model, const SysView& s,
+                 const MixedBuffers& b, const TripList& T, const StageKeep& KS, bool merge_sf, hipStream_t stream);
+void launch_force32(const MixedModel& mm, const ModelT& t, const ModelT* d_model, const SysView& s,
+                    const MixedBuffers& b, const TripList& T, const StageKeep& KS, bool merge_f, bool push,
+                    hipStream_t stream);
 // Tangent of the scaled SFs along a displacement field u [3N]:
 // Gdot[i*ldG + q] = sum_a dG_iq/dx_a . u_a, recomputed in FP32.
 void launch_tangent32(const MixedModel& mm, const ModelT& t, const ModelT* d_model, const SysView& s,

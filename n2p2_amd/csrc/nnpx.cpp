@@ -821,7 +821,7 @@ MixedBuffers mixed_buffers(nnpx_ctx* c)
         m.trips.cap = c->trip_cap;
         m.trips.ld = c->mixed.max_walks;
         m.trips.list = buf<unsigned>(c, "trips", tl);
-        m.trips.counts = buf<int>(c, "trip_n", (size_t)c->N * m.trips.ld);
+        m.trips.counts = buf<int>(c, "trip_n", (size_t)c->N * kListWaves * m.trips.ld);
     }
     return m;
 }
@@ -2015,7 +2015,7 @@ nnpx_status nnpx_autotune(nnpx_ctx* c)
         const int capL = c->cap;
         const ModelT& t = c->hm.t;
         auto fits = [&](int trip, size_t extra) {
-            return stage_bytes(capL, trip, stage_mp(0, 0)) + extra <= 65536;
+            return stage_bytes(capL, 1, trip, stage_mp(0, 0, 1)) + extra <= 65536;
         };
         c->timing = true;
         double best_t = 1e30;
