@@ -65,6 +65,10 @@ void fill_int(int* p, int v, size_t n, hipStream_t stream, const int* gate = nul
 // and order).
 // clear_flags: reset the overflow flags first (MD keeps them across rebuilds).
 void launch_neighbors(const SysView& s, double rc, bool any_cell, hipStream_t stream, bool clear_flags = true);
+// A caller's packed neighbour entries (atom i's are off[i] .. off[i + 1] - 1)
+// spread to the list's rows: counts, indices, image `img` and vectors.
+void launch_spread_entries(const SysView& s, const int64_t* off, const int* index, const double* dr, int img,
+                           double* nb_dr, hipStream_t stream);
 // Reverse entries: for (i -> j, image) the slot of (j -> i, -image).
 void launch_reverse(const SysView& s, hipStream_t stream);
 

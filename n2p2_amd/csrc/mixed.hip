@@ -285,6 +285,53 @@ int pow2_exponent(double zeta)
 
 }  // namespace
 
+static void pack_weights(MixedModel& mm, const HostModel& hm, std::vector<uint16_t>& w, std::vector<float>& b)
+{
+    // bf16 weights, padded to 16: W [out][in] and WT [in][out], hi then lo.
+    const ModelT& t = hm.t;
+    w.clear();
+    b.clear();
+    auto pad16 = [](int x) { return (x + 15) / 16 * 16; };
+    mm.maxpad = 16;
+    mm.maxpadh = 16;
+    mm.ldK = 16;
+    for (int e = 0; e < t.nelem; ++e) {
+        const NNT& N = t.el[e].nn;
+        mm.ldK = std::max(mm.ldK, pad16(N.n[0]));
+        for (int l = 1; l < N.nl; ++l) {
+            const int nin = N.n[l - 1], nout = N.n[l];
+            const int pi = pad16(nin), po = pad16(nout);
+            mm.pin[e][l] = pi;
+            mm.pout[e][l] = po;
+            mm.maxpad = std::max(mm.maxpad, std::max(pi, po));
+            mm.maxpadh = std::max(mm.maxpadh, po);
+            std::vector<float> W((size_t)po * pi, 0.f);
+            for (int k = 0; k < nout; ++k)
+                for (int j = 0; j < nin; ++j) W[(size_t)k * pi + j] = (float)hm.weights[N.woff[l] + (size_t)k * nin + j];
+            mm.wW[e][l] = (int)w.size();
+            std::vector<uint16_t> hi(W.size()), lo(W.size());
+            for (size_t q = 0; q < W.size(); ++q) {
+                hi[q] = to_bf16(W[q]);
+                lo[q] = to_bf16(W[q] - from_bf16(hi[q]));
+            }
+            w.insert(w.end(), hi.begin(), hi.end());
+            w.insert(w.end(), lo.begin(), lo.end());
+            mm.wT[e][l] = (int)w.size();
+            for (int j = 0; j < pi; ++j)
+                for (int k = 0; k < po; ++k) hi[(size_t)j * po + k] = to_bf16(W[(size_t)k * pi + j]);
+            for (int j = 0; j < pi; ++j)
+                for (int k = 0; k < po; ++k) {
+                    const float x = W[(size_t)k * pi + j];
+                    lo[(size_t)j * po + k] = to_bf16(x - from_bf16(to_bf16(x)));
+                }
+            w.insert(w.end(), hi.begin(), hi.end());
+            w.insert(w.end(), lo.begin(), lo.end());
+            mm.bo[e][l] = (int)b.size();
+            for (int k = 0; k < po; ++k) b.push_back(k < nout ? (float)hm.weights[N.boff[l] + k] : 0.f);
+        }
+    }
+}
+
 void setup_mixed(MixedModel& mm, const HostModel& hm)
 {
     free_mixed(mm);
@@ -473,48 +520,9 @@ void setup_mixed(MixedModel& mm, const HostModel& hm)
         }
         mm.max_walks = std::max(mm.max_walks, nw);
     }
-    // bf16 weights, padded to 16: W [out][in] and WT [in][out], hi then lo.
     std::vector<uint16_t> w;
     std::vector<float> b;
-    auto pad16 = [](int x) { return (x + 15) / 16 * 16; };
-    mm.maxpad = 16;
-    mm.maxpadh = 16;
-    mm.ldK = 16;
-    for (int e = 0; e < t.nelem; ++e) {
-        const NNT& N = t.el[e].nn;
-        mm.ldK = std::max(mm.ldK, pad16(N.n[0]));
-        for (int l = 1; l < N.nl; ++l) {
-            const int nin = N.n[l - 1], nout = N.n[l];
-            const int pi = pad16(nin), po = pad16(nout);
-            mm.pin[e][l] = pi;
-            mm.pout[e][l] = po;
-            mm.maxpad = std::max(mm.maxpad, std::max(pi, po));
-            mm.maxpadh = std::max(mm.maxpadh, po);
-            std::vector<float> W((size_t)po * pi, 0.f);
-            for (int k = 0; k < nout; ++k)
-                for (int j = 0; j < nin; ++j) W[(size_t)k * pi + j] = (float)hm.weights[N.woff[l] + (size_t)k * nin + j];
-            mm.wW[e][l] = (int)w.size();
-            std::vector<uint16_t> hi(W.size()), lo(W.size());
-            for (size_t q = 0; q < W.size(); ++q) {
-                hi[q] = to_bf16(W[q]);
-                lo[q] = to_bf16(W[q] - from_bf16(hi[q]));
-            }
-            w.insert(w.end(), hi.begin(), hi.end());
-            w.insert(w.end(), lo.begin(), lo.end());
-            mm.wT[e][l] = (int)w.size();
-            for (int j = 0; j < pi; ++j)
-                for (int k = 0; k < po; ++k) hi[(size_t)j * po + k] = to_bf16(W[(size_t)k * pi + j]);
-            for (int j = 0; j < pi; ++j)
-                for (int k = 0; k < po; ++k) {
-                    const float x = W[(size_t)k * pi + j];
-                    lo[(size_t)j * po + k] = to_bf16(x - from_bf16(to_bf16(x)));
-                }
-            w.insert(w.end(), hi.begin(), hi.end());
-            w.insert(w.end(), lo.begin(), lo.end());
-            mm.bo[e][l] = (int)b.size();
-            for (int k = 0; k < po; ++k) b.push_back(k < nout ? (float)hm.weights[N.boff[l] + k] : 0.f);
-        }
-    }
+    pack_weights(mm, hm, w, b);
     auto up = [](void** dst, const void* src, size_t bytes) {
         if (hipMalloc(dst, std::max<size_t>(bytes, 16)) != hipSuccess) throw Error{NNPX_ERR_HIP, "hipMalloc mixed"};
         if (hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice) != hipSuccess) throw Error{NNPX_ERR_HIP, "hipMemcpy"};
@@ -527,6 +535,19 @@ void setup_mixed(MixedModel& mm, const HostModel& hm)
     up((void**)&mm.d_w, w.data(), sizeof(uint16_t) * w.size());
     up((void**)&mm.d_b, b.data(), sizeof(float) * b.size());
     mm.ready = true;
+}
+
+// New weights for the model that setup_mixed() saw: the networks' tables keep
+// their sizes, nothing else depends on the weights.
+void update_mixed_weights(MixedModel& mm, const HostModel& hm)
+{
+    if (!mm.ready) throw Error{NNPX_ERR_STATE, "mixed-precision tables not set up"};
+    std::vector<uint16_t> w;
+    std::vector<float> b;
+    pack_weights(mm, hm, w, b);
+    if (hipMemcpy(mm.d_w, w.data(), sizeof(uint16_t) * w.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(mm.d_b, b.data(), sizeof(float) * b.size(), hipMemcpyHostToDevice) != hipSuccess)
+        throw Error{NNPX_ERR_HIP, "hipMemcpy"};
 }
 
 void free_mixed(MixedModel& mm)

@@ -178,6 +178,7 @@ struct MixedBuffers {
 using TimedFn = std::function<void(const char*, const std::function<void()>&)>;
 
 void setup_mixed(MixedModel& mm, const HostModel& hm);
+void update_mixed_weights(MixedModel& mm, const HostModel& hm);
 void free_mixed(MixedModel& mm);
 void run_mixed(const MixedModel& mm, const ModelT& t, const ModelT* d_model, const SysView& s,
                const MixedBuffers& b, bool forces, bool push, hipStream_t stream, const TimedFn& timed);

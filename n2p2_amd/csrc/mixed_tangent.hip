@@ -18,7 +18,7 @@ namespace {
 // x, y shared by the terms; terms summed over a buffer in FP32, then folded
 // into compensated sums, as the values are.  Bound by instruction issue like
 // the force kernel; 41,000 atoms, 30 angular functions per element: 1,342 us
-// with an exponential and a logarithm's share per member, 880 us so.
+// with an exponential per member, 939 us so.
 template <int W, int MAXM, bool FAST, int NB0, int NB1, bool COS>
 __global__ __launch_bounds__(W * kWave) void k_tangent32(const ModelT* __restrict__ M, const MemberF* __restrict__ MF,
                                                          const GroupMixF* __restrict__ GM, SysView s,

@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <string>
@@ -63,7 +64,12 @@ struct Timer {
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    bool part = false;  // a piece of the input block, not an allocation of its own
 };
+
+// Arrays up to this size pass through a context's pinned host memory (several
+// to a transfer, no wait for each); larger ones are copied where they are.
+constexpr size_t kPinnedArray = (size_t)256 << 10;
 
 }  // namespace
 
@@ -103,6 +109,12 @@ struct nnpx_ctx {
     int md_stage_req = -1;       // NNPX_OPT_MD_STAGING
     bool nbr_valid = false;
     bool rev_valid = false;
+    // setting the structures builds their list (it sizes the capacity): the
+    // first evaluation of those positions takes that list
+    bool list_fresh = false;
+    bool settled = false;        // the flags of the work so far were read and clear
+    // pinned host memory for small transfers (inputs; results and flags)
+    DevBuf pin_in, pin_out;
     // results state
     bool sf_valid = false, sfd_valid = false, nn_valid = false, dedg_valid = false;
     // the plain gradient calls leave dG/dr to be had like the results: it is
@@ -211,6 +223,7 @@ T* buf(nnpx_ctx* c, const std::string& name, size_t count)
         return static_cast<T*>(a.p);
     }
     DevBuf& b = c->bufs[name];
+    if (b.part) b = DevBuf{};  // an allocation of its own again
     if (b.bytes < bytes) {
         drop_graph(c);
         if (b.p) hip_check(hipFree(b.p), "hipFree");
@@ -220,6 +233,20 @@ T* buf(nnpx_ctx* c, const std::string& name, size_t count)
         b.bytes = bytes;
     }
     return static_cast<T*>(b.p);
+}
+
+// Pinned host memory of at least `bytes` (kept by the context).
+unsigned char* pinned(DevBuf& b, size_t bytes)
+{
+    if (b.bytes < bytes) {
+        if (b.p) hip_check(hipHostFree(b.p), "hipHostFree");
+        b.p = nullptr;
+        b.bytes = 0;
+        const size_t want = std::max<size_t>(bytes, 4096);
+        hip_check(hipHostMalloc(&b.p, want), "hipHostMalloc");
+        b.bytes = want;
+    }
+    return static_cast<unsigned char*>(b.p);
 }
 
 // Model-level tables (set up with the model, read by the kernels of every
@@ -238,6 +265,51 @@ T* existing(nnpx_ctx* c, const std::string& name)
     auto& m = c->arena ? c->abufs : c->bufs;
     auto it = m.find(name);
     return it == m.end() ? nullptr : static_cast<T*>(it->second.p);
+}
+
+struct Upload {
+    const char* name;
+    const void* src;
+    size_t bytes;
+};
+
+// Copies host arrays to the named buffers.  They lie in one block; the small
+// ones go in one transfer from pinned memory.  The stream must be idle (the
+// pinned memory and the block are reused).
+void upload(nnpx_ctx* c, std::initializer_list<Upload> list)
+{
+    if (c->arena) {
+        for (const Upload& u : list) {
+            char* d = buf<char>(c, u.name, u.bytes);
+            if (u.bytes) hip_check(hipMemcpy(d, u.src, u.bytes, hipMemcpyHostToDevice), "hipMemcpy");
+        }
+        return;
+    }
+    auto pad = [](size_t n) { return (n + 255) / 256 * 256; };
+    size_t small = 0, total = 0;
+    for (const Upload& u : list) {
+        total += pad(u.bytes);
+        if (u.bytes <= kPinnedArray) small += pad(u.bytes);
+    }
+    // no piece outlives its block, also where the next one cannot be had
+    for (auto& kv : c->bufs)
+        if (kv.second.part) kv.second = DevBuf{};
+    char* block = buf<char>(c, "in_block", total);
+    unsigned char* pin = pinned(c->pin_in, small);
+    size_t at = 0, big = small;  // small pieces first, as they lie in the pinned memory
+    for (const Upload& u : list) {
+        DevBuf& b = c->bufs[u.name];
+        if (b.p) hip_check(hipFree(b.p), "hipFree");
+        size_t& off = u.bytes <= kPinnedArray ? at : big;
+        b.p = block + off;
+        b.bytes = u.bytes;
+        b.part = true;
+        if (u.bytes == 0) continue;
+        if (u.bytes <= kPinnedArray) std::memcpy(pin + off, u.src, u.bytes);
+        else hip_check(hipMemcpy(b.p, u.src, u.bytes, hipMemcpyHostToDevice), "hipMemcpy");
+        off += pad(u.bytes);
+    }
+    if (small) hip_check(hipMemcpyAsync(block, pin, small, hipMemcpyHostToDevice, c->stream), "hipMemcpyAsync");
 }
 
 hipEvent_t get_event(nnpx_ctx* c)
@@ -336,6 +408,7 @@ void need_structures(nnpx_ctx* c)
 
 void invalidate(nnpx_ctx* c)
 {
+    c->settled = false;
     c->sf_valid = c->sfd_valid = c->nn_valid = c->dedg_valid = c->e_valid = c->f_valid = false;
     c->dgdr_due = false;
 }
@@ -470,9 +543,11 @@ void alloc_neighbors(nnpx_ctx* c)
 // entries, most angular pairs per atom.
 void read_flags(nnpx_ctx* c, int (&f)[4])
 {
-    hip_check(hipMemcpyAsync(f, existing<int>(c, "flags"), 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream),
+    int* dst = c->arena ? f : reinterpret_cast<int*>(pinned(c->pin_out, sizeof f));
+    hip_check(hipMemcpyAsync(dst, existing<int>(c, "flags"), sizeof f, hipMemcpyDeviceToHost, c->stream),
               "hipMemcpyAsync");
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    if (dst != f) std::memcpy(f, dst, sizeof f);
 }
 
 // Sizes the angular pair lists for the most pairs per atom of the last
@@ -493,10 +568,12 @@ void build_neighbors(nnpx_ctx* c, bool check)
         c->nbr_valid = true;
         return;
     }
+    c->list_fresh = false;
     for (int attempt = 0; attempt < 3; ++attempt) {
         alloc_neighbors(c);
         SysView s = sysview(c);
         timed(c, "nbr", [&] { launch_neighbors(s, list_cutoff(c), c->any_cell, c->stream); });
+        c->settled = false;
         c->rev_valid = false;
         if (!check) break;
         int f[4];
@@ -511,8 +588,9 @@ void build_neighbors(nnpx_ctx* c, bool check)
 }
 
 // FP64 weights in model layout followed by a transposed copy ([in][out]),
-// and the BF16/FP32 tables of the mixed form.
-void upload_weights(nnpx_ctx* c)
+// and the BF16/FP32 tables of the mixed form (all of them for a new model, the
+// networks' alone for new weights of the same one).
+void upload_weights(nnpx_ctx* c, bool new_model)
 {
     const ModelT& t = c->hm.t;
     std::vector<double> w2(2 * (size_t)t.nweights, 0.0);
@@ -527,7 +605,8 @@ void upload_weights(nnpx_ctx* c)
     }
     if (!c->d_w) hip_check(hipMalloc(&c->d_w, sizeof(double) * w2.size()), "hipMalloc weights");
     hip_check(hipMemcpy(c->d_w, w2.data(), sizeof(double) * w2.size(), hipMemcpyHostToDevice), "hipMemcpy");
-    setup_mixed(c->mixed, c->hm);
+    if (new_model || !c->mixed.ready) setup_mixed(c->mixed, c->hm);
+    else update_mixed_weights(c->mixed, c->hm);
 }
 
 // Connections per element in NeuralNetwork::setConnections order
@@ -565,6 +644,7 @@ void compute_sf64(nnpx_ctx* c, bool deriv)
     }
     c->sf_valid = true;
     c->sfd_valid = deriv;
+    c->settled = false;
 }
 
 void compute_nn64(nnpx_ctx* c, bool deriv)
@@ -581,6 +661,7 @@ void compute_nn64(nnpx_ctx* c, bool deriv)
     });
     c->nn_valid = true;
     c->dedg_valid = deriv;
+    c->settled = false;
 }
 
 // Whether dG/dr is stored, storing it first where a gradient call left it due.
@@ -606,6 +687,7 @@ void compute_force64_fused(nnpx_ctx* c)
                              c->external || c->force_mode == NNPX_FORCES_PUSH, c->stream);
     });
     c->f_valid = true;
+    c->settled = false;
 }
 
 // The fused FP64 force kernel stages the whole list in LDS.
@@ -616,10 +698,12 @@ void compute_energy(nnpx_ctx* c)
     double* E = buf<double>(c, "E", c->S);
     timed(c, "energy", [&] { launch_energy(existing<double>(c, "Eatom"), existing<int>(c, "atom_off"), c->S, E, c->stream); });
     c->e_valid = true;
+    c->settled = false;
 }
 
 void compute_force64(nnpx_ctx* c)
 {
+    c->settled = false;
     const ModelT& t = c->hm.t;
     double* f = buf<double>(c, "F", (size_t)3 * force_entries(c));
     SysView s = sysview(c);
@@ -658,7 +742,8 @@ void evaluate(nnpx_ctx* c, int precision, unsigned flags, bool check, bool store
                 existing<StructT>(c, "st"), c->N, gate, c->stream);
         md_set_gate(gate, 0, c->stream);
     }
-    build_neighbors(c, check);
+    if (c->list_fresh && !c->md_ready) c->list_fresh = false;
+    else build_neighbors(c, check);
     // an external list has no build kernel to clear the flags the mixed
     // kernels set
     if (c->external) fill_int(existing<int>(c, "flags"), 0, 4, c->stream);
@@ -690,6 +775,7 @@ void evaluate(nnpx_ctx* c, int precision, unsigned flags, bool check, bool store
 // was checked; an overflow re-runs the evaluation with a larger capacity.
 void settle(nnpx_ctx* c)
 {
+    if (c->settled) return;
     int f[4];
     read_flags(c, f);
     fit_trips(c, f[3]);
@@ -702,12 +788,12 @@ void settle(nnpx_ctx* c)
         // checked rebuild refits the staging capacity to this list
         evaluate(c, c->last_precision, c->f_valid ? NNPX_EVAL_FORCES : 0u, true, c->last_stored);
     } else {
-        hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        c->settled = true;  // read_flags waited for the stream
         return;
     }
     read_flags(c, f);
     if (f[0] & 7) fail(NNPX_ERR_HIP, "neighbour list or staging overflow persists after a refit");
-    hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    c->settled = true;
 }
 
 // Structures of nnpx_set_structures (copied to device buffers; the first
@@ -725,6 +811,7 @@ void set_structures(nnpx_ctx* c, int ns, const int64_t* off, const double* pos, 
     // a new structure set ends any MD set-up (skin, graph) and any
     // caller-provided neighbour list
     c->external = false;
+    c->list_fresh = false;
     c->ntotal = 0;
     c->skin = 0.0;
     c->md_ready = false;
@@ -759,16 +846,12 @@ void set_structures(nnpx_ctx* c, int ns, const int64_t* off, const double* pos, 
     }
     std::vector<int> off32(ns + 1);
     for (int s = 0; s <= ns; ++s) off32[s] = (int)off[s];
-    auto up = [&](const std::string& name, const void* src, size_t bytes) {
-        void* d = buf<char>(c, name, bytes);
-        hip_check(hipMemcpy(d, src, bytes, hipMemcpyHostToDevice), "hipMemcpy");
-    };
-    up("pos", pos, sizeof(double) * 3 * N);
-    up("elem", elem, sizeof(int) * N);
-    up("sid", sid.data(), sizeof(int) * N);
-    up("st", c->st_host.data(), sizeof(StructT) * ns);
-    up("elem_atoms", atoms.data(), sizeof(int) * N);
-    up("atom_off", off32.data(), sizeof(int) * (ns + 1));
+    upload(c, {{"pos", pos, sizeof(double) * 3 * N},
+               {"elem", elem, sizeof(int) * N},
+               {"sid", sid.data(), sizeof(int) * N},
+               {"st", c->st_host.data(), sizeof(StructT) * ns},
+               {"elem_atoms", atoms.data(), sizeof(int) * N},
+               {"atom_off", off32.data(), sizeof(int) * (ns + 1)}});
     c->cap = estimate_cap(c);
     c->nbr_valid = false;
     invalidate(c);
@@ -777,14 +860,48 @@ void set_structures(nnpx_ctx* c, int ns, const int64_t* off, const double* pos, 
     const int want = ((c->max_nb + c->max_nb / 8 + 8 + 31) / 32) * 32;
     if (want < c->cap) {
         c->cap = std::max(want, 32);
-        build_neighbors(c, true);
+        build_neighbors(c, false);  // the counts are known to fit
     }
+    c->list_fresh = true;
 }
 
 void copy_out(nnpx_ctx* c, void* dst, const void* src, size_t bytes)
 {
-    hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync");
+    if (c->arena || bytes > kPinnedArray) {
+        hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync");
+        hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        return;
+    }
+    unsigned char* pin = pinned(c->pin_out, bytes);
+    hip_check(hipMemcpyAsync(pin, src, bytes, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync");
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    std::memcpy(dst, pin, bytes);
+}
+
+// A result of the settled evaluation: the flags come in the same wait as the
+// result, which is read again only if they ask for a repeat.
+void get_result(nnpx_ctx* c, void* dst, const char* name, size_t bytes)
+{
+    if (c->arena || c->settled || bytes > kPinnedArray) {
+        settle(c);
+        copy_out(c, dst, existing<char>(c, name), bytes);
+        return;
+    }
+    unsigned char* pin = pinned(c->pin_out, bytes + 16);
+    hip_check(hipMemcpyAsync(pin, existing<int>(c, "flags"), 16, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync");
+    hip_check(hipMemcpyAsync(pin + 16, existing<char>(c, name), bytes, hipMemcpyDeviceToHost, c->stream),
+              "hipMemcpyAsync");
+    hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    int f[4];
+    std::memcpy(f, pin, sizeof f);
+    if (f[0] & 7) {
+        settle(c);
+        copy_out(c, dst, existing<char>(c, name), bytes);
+        return;
+    }
+    fit_trips(c, f[3]);
+    c->settled = true;
+    std::memcpy(dst, pin + 16, bytes);
 }
 
 }  // namespace
@@ -866,7 +983,9 @@ nnpx_status nnpx_destroy(nnpx_ctx* c)
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     for (auto& kv : c->bufs)
-        if (kv.second.p) (void)hipFree(kv.second.p);
+        if (kv.second.p && !kv.second.part) (void)hipFree(kv.second.p);
+    if (c->pin_in.p) (void)hipHostFree(c->pin_in.p);
+    if (c->pin_out.p) (void)hipHostFree(c->pin_out.p);
     if (c->d_model) (void)hipFree(c->d_model);
     if (c->d_w) (void)hipFree(c->d_w);
     free_mixed(c->mixed);
@@ -979,7 +1098,7 @@ nnpx_status nnpx_load_model(nnpx_ctx* c, const char* dir)
         hip_check(hipMemcpy(c->d_model, &t, sizeof(ModelT), hipMemcpyHostToDevice), "hipMemcpy model");
         if (c->d_w) hip_check(hipFree(c->d_w), "hipFree");
         c->d_w = nullptr;
-        upload_weights(c);
+        upload_weights(c, true);
         // SF -> derivative slot per (centre element, neighbour element)
         std::vector<int> islot((size_t)kMaxElem * kMaxElem * kMaxSF, -1);
         for (int e = 0; e < t.nelem; ++e)
@@ -1131,6 +1250,7 @@ nnpx_status nnpx_set_neighbors_external(nnpx_ctx* c, int nlocal, const int* elem
         c->md_ready = false;
         c->skin = 0.0;
         c->external = true;
+        c->list_fresh = false;
         c->ntotal = ntotal;
         c->N = nlocal;
         c->S = 1;
@@ -1153,34 +1273,31 @@ nnpx_status nnpx_set_neighbors_external(nnpx_ctx* c, int nlocal, const int* elem
         c->cap = std::max(32, ((maxn + 31) / 32) * 32);
         c->max_nb = maxn;
         c->stage_cap = 0;  // stage the whole list (a fit from earlier structures does not apply)
+        // the caller's packed entries as they are, spread to the list's rows by
+        // a kernel
         const size_t slots = (size_t)nlocal * c->cap;
-        std::vector<int> nn(nlocal), jj(slots, 0), im(slots, pack_image(0, 0, 0));
-        std::vector<double> dr(3 * slots, 0.0);
-        for (int i = 0; i < nlocal; ++i) {
-            nn[i] = (int)(nb_offsets[i + 1] - nb_offsets[i]);
-            for (int k = 0; k < nn[i]; ++k) {
-                const int64_t p = nb_offsets[i] + k;
-                jj[(size_t)i * c->cap + k] = nb_index[p];
-                for (int x = 0; x < 3; ++x) dr[3 * ((size_t)i * c->cap + k) + x] = nb_dr[3 * p + x];
-            }
-        }
-        std::vector<int> sid(nlocal, 0), off32 = {0, nlocal}, flags(4, 0);
+        std::vector<int> sid(nlocal, 0), off32 = {0, nlocal};
         std::vector<double> pos(3 * (size_t)nlocal, 0.0);
-        auto up = [&](const std::string& name, const void* src, size_t bytes) {
-            void* d = buf<char>(c, name, bytes);
-            hip_check(hipMemcpy(d, src, bytes, hipMemcpyHostToDevice), "hipMemcpy");
-        };
-        up("pos", pos.data(), sizeof(double) * pos.size());
-        up("elem", el_all.data(), sizeof(int) * ntotal);
-        up("sid", sid.data(), sizeof(int) * nlocal);
-        up("st", c->st_host.data(), sizeof(StructT));
-        up("elem_atoms", atoms.data(), sizeof(int) * nlocal);
-        up("atom_off", off32.data(), sizeof(int) * 2);
-        up("nb_n", nn.data(), sizeof(int) * nlocal);
-        up("nb_j", jj.data(), sizeof(int) * slots);
-        up("nb_img", im.data(), sizeof(int) * slots);
-        up("nb_dr", dr.data(), sizeof(double) * dr.size());
-        up("flags", flags.data(), sizeof(int) * flags.size());
+        upload(c, {{"pos", pos.data(), sizeof(double) * pos.size()},
+                   {"elem", el_all.data(), sizeof(int) * ntotal},
+                   {"sid", sid.data(), sizeof(int) * nlocal},
+                   {"st", c->st_host.data(), sizeof(StructT)},
+                   {"elem_atoms", atoms.data(), sizeof(int) * nlocal},
+                   {"atom_off", off32.data(), sizeof(int) * 2},
+                   {"x_off", nb_offsets, sizeof(int64_t) * (nlocal + 1)},
+                   {"x_index", nb_index, sizeof(int) * P},
+                   {"x_dr", nb_dr, sizeof(double) * 3 * P}});
+        SysView s{};
+        s.natoms = nlocal;
+        s.cap = c->cap;
+        s.nb_n = buf<int>(c, "nb_n", nlocal);
+        s.nb_j = buf<int>(c, "nb_j", slots);
+        s.nb_img = buf<int>(c, "nb_img", slots);
+        launch_spread_entries(s, existing<int64_t>(c, "x_off"), existing<int>(c, "x_index"),
+                              existing<double>(c, "x_dr"), pack_image(0, 0, 0), buf<double>(c, "nb_dr", 3 * slots),
+                              c->stream);
+        hip_check(hipGetLastError(), "spread");
+        fill_int(buf<int>(c, "flags", 4), 0, 4, c->stream);
         buf<int>(c, "nb_rev", slots);
         invalidate(c);
         c->nbr_valid = true;
@@ -1214,8 +1331,16 @@ nnpx_status nnpx_update_positions(nnpx_ctx* c, const double* pos)
             hip_check(hipMemcpy(existing<StructT>(c, "st"), c->st_host.data(), sizeof(StructT) * c->S,
                                 hipMemcpyHostToDevice),
                       "hipMemcpy");
-        hip_check(hipMemcpy(existing<double>(c, "pos"), pos, sizeof(double) * 3 * c->N, hipMemcpyHostToDevice),
-                  "hipMemcpy");
+        const size_t bytes = sizeof(double) * 3 * c->N;
+        if (bytes <= kPinnedArray) {
+            unsigned char* pin = pinned(c->pin_in, bytes);
+            std::memcpy(pin, pos, bytes);
+            hip_check(hipMemcpyAsync(existing<double>(c, "pos"), pin, bytes, hipMemcpyHostToDevice, c->stream),
+                      "hipMemcpyAsync");
+        } else {
+            hip_check(hipMemcpy(existing<double>(c, "pos"), pos, bytes, hipMemcpyHostToDevice), "hipMemcpy");
+        }
+        c->list_fresh = false;
         c->nbr_valid = false;
         invalidate(c);
     });
@@ -1226,7 +1351,8 @@ nnpx_status nnpx_calculate_neighbor_list(nnpx_ctx* c)
     return guard(c, [&] {
         need_structures(c);
         invalidate(c);
-        build_neighbors(c, true);
+        if (c->list_fresh) c->list_fresh = false;
+        else build_neighbors(c, true);
     });
 }
 
@@ -1286,8 +1412,7 @@ nnpx_status nnpx_get_energy(nnpx_ctx* c, double* E)
         need_structures(c);
         if (!E) fail(NNPX_ERR_ARGUMENT, "null output");
         if (!c->e_valid) fail(NNPX_ERR_STATE, "energy not calculated");
-        settle(c);
-        copy_out(c, E, existing<double>(c, "E"), sizeof(double) * c->S);
+        get_result(c, E, "E", sizeof(double) * c->S);
     });
 }
 
@@ -1297,8 +1422,7 @@ nnpx_status nnpx_get_atomic_energies(nnpx_ctx* c, double* e)
         need_structures(c);
         if (!e) fail(NNPX_ERR_ARGUMENT, "null output");
         if (!c->nn_valid) fail(NNPX_ERR_STATE, "atomic neural networks not calculated");
-        settle(c);
-        copy_out(c, e, existing<double>(c, "Eatom"), sizeof(double) * c->N);
+        get_result(c, e, "Eatom", sizeof(double) * c->N);
     });
 }
 
@@ -1308,8 +1432,7 @@ nnpx_status nnpx_get_forces(nnpx_ctx* c, double* f)
         need_structures(c);
         if (!f) fail(NNPX_ERR_ARGUMENT, "null output");
         if (!c->f_valid) fail(NNPX_ERR_STATE, "forces not calculated");
-        settle(c);
-        copy_out(c, f, existing<double>(c, "F"), sizeof(double) * 3 * force_entries(c));
+        get_result(c, f, "F", sizeof(double) * 3 * force_entries(c));
     });
 }
 
@@ -1584,7 +1707,7 @@ void set_connections(nnpx_ctx* c, const double* w)
             for (int k = 0; k < N.n[l]; ++k) c->hm.weights[N.boff[l] + k] = w[p++];
         }
     }
-    upload_weights(c);
+    upload_weights(c, false);
     drop_graph(c);
     invalidate(c);
 }
@@ -2396,6 +2519,7 @@ void md_steps(nnpx_ctx* c, int nsteps, int graph_steps)
         int f[4];
         read_flags(c, f);
         if (f[0] & 1) fail(NNPX_ERR_RANGE, "neighbour capacity exceeded during MD (raise the skin or re-initialise)");
+        c->settled = false;
         c->sf_valid = c->nn_valid = c->dedg_valid = c->e_valid = c->f_valid = true;
         c->sfd_valid = c->md_precision == NNPX_PLAIN_FP64 && !fused_fits(c);
         c->last_stored = c->sfd_valid;
