@@ -249,6 +249,14 @@ __device__ inline T lane_value(T v, int l)
     }
 }
 
+// Orders a wave's LDS writes before its own later reads (the hardware keeps a
+// wave's LDS accesses in order; this keeps the compiler from moving them).
+__device__ inline void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Sum over the wave, received by every lane: pairwise sums inside rows of 16
 // (quad swaps, half-row and row mirrors), then the four row sums added in
 // row order.

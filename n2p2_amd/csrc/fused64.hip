@@ -102,14 +102,6 @@ __host__ __device__ constexpr size_t stage64_bytes(int capL, int waves, int walk
            (size_t)waves * (walk + kWave) * 4 + 48;
 }
 
-// Orders a wave's LDS writes before its own later reads (the hardware keeps a
-// wave's LDS accesses in order; this keeps the compiler from moving them).
-__device__ inline void wave_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 template <int W>
 __device__ inline Stage64 carve64(double4* base, int capL, int walk)
 {

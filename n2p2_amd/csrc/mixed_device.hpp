@@ -323,14 +323,6 @@ struct NoFlush {
     __device__ void operator()() const {}
 };
 
-// Orders a wave's LDS writes before its own later reads (the hardware keeps a
-// wave's LDS accesses in order; this keeps the compiler from moving them).
-__device__ inline void wave_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Runs `work` over the first cnt buffered pairs, each lane a contiguous
 // chunk, so a lane sees runs of one first atom j (j's geometry stays in
 // registers over the run and the force kernel keeps j's contribution there).
