@@ -259,8 +259,8 @@ nnpx_status nnpx_set_weights(nnpx_ctx* ctx, const double* w);
  * loss[0] = L, loss[1] = energy term, loss[2] = force term.  The force term
  * is differentiated through the forces (second order) as Training::dPdc
  * with NeuralNetwork::calculateDFdc and Training::collectDGdxia do
- * (Training.cpp:3319-3389, 3586-3625).  NNPX_PLAIN_FP64: FP64 from the stored
- * dG/dr; NNPX_MIXED: FP32 recomputed tangents and FP32 network adjoints,
+ * (Training.cpp:3319-3389, 3586-3625).  NNPX_PLAIN_FP64: FP64 recomputed
+ * tangents (from the stored dG/dr where an evaluation keeps it); NNPX_MIXED: FP32 recomputed tangents and FP32 network adjoints,
  * gradient summed in FP64.  Model units; normalize_nodes is not supported. */
 nnpx_status nnpx_loss_gradient(nnpx_ctx* ctx, int precision, const double* E_ref,
                                const double* F_ref, double beta, double* loss,
@@ -338,7 +338,7 @@ nnpx_status nnpx_md_energies(nnpx_ctx* ctx, double* epot, double* ekin,
 /* No counterpart in the reference.  Times candidate launch shapes of the
  * mixed-form kernels on the current structures (HIP events, 3 launches
  * each) and keeps the fastest in the context: the triplet-buffer size of the
- * SF, force and tangent kernels (LDS per wave against batching) and the
+ * SF, force and tangent kernels (per wave: LDS against batching) and the
  * atoms per block of the gradient kernel.  Results are not changed by the
  * choice beyond summation order.  values[4] = {trip_sf, trip_force,
  * trip_tangent, grad_atoms}; triplet buffers are multiples of 64 in
