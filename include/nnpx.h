@@ -96,9 +96,9 @@ typedef enum {
                                   and the force kernel reads them instead
                                   of testing the candidates again (both
                                   walk row x column blocks); off, the
-                                  force kernel walks rows.  -1 auto (off
-                                  until nnpx_autotune keeps the faster,
-                                  default), 0 off, 1 on; results agree to
+                                  force kernel walks rows.  -1 auto (on
+                                  from 1,024 atoms, until nnpx_autotune
+                                  keeps the faster; default), 0 off, 1 on; results agree to
                                   FP32 summation order                     */
 } nnpx_option;
 

@@ -593,13 +593,15 @@ void run_mixed(const MixedModel& mm, const ModelT& t, const ModelT* d_model, con
     // kernel when both make the same walks (the SF kernel also counts them,
     // which sizes the lists of later evaluations); off, the force kernel
     // walks rows
-    const bool lists = mm.tune.pair_lists == 1;
+    const bool lists = keep_lists(mm.tune, s.natoms);
     TripList T{};
     if (forces && lists && merge_sf == merge_f) {
         T = b.trips;
         T.count = true;
     }
-    T.rows = !lists;
+    // lists not set by the caller and not there (the first evaluation only counts
+    // the pairs): rows, the faster walk of the two
+    T.rows = !lists || (mm.tune.pair_lists < 0 && !T.list);
     // the staging passes from the SF to the force kernel (identical values)
     const StageKeep KS = forces && b.keep.ld >= capL ? b.keep : StageKeep{};
     // a model of compact functions alone leaves these kernels nothing: its

@@ -126,7 +126,7 @@ struct Tuning {
     int sf_gather = -1;      // SF kernel partner gather: -1 auto, 0 off, 1 on
     int merge_sf = -1;       // merged angular walk in the SF kernel: -1 auto, 0 off, 1 on
     int merge_force = -1;    // ... in the force kernel
-    int pair_lists = -1;     // angular pair lists from the SF to the force kernel: -1 auto (off until tuned), 0 off, 1 on
+    int pair_lists = -1;     // angular pair lists from the SF to the force kernel: -1 by the atom count (keep_lists), 0 off, 1 on
 };
 
 struct MixedModel {
@@ -177,6 +177,18 @@ struct MixedBuffers {
 
 using TimedFn = std::function<void(const char*, const std::function<void()>&)>;
 
+// Whether the SF kernel keeps the angular pairs for the force kernel: as set, or
+// from 1,024 atoms on, where an atom has at most two waves and testing its
+// candidates again costs more than the lists' traffic.  Values + forces in us
+// without and with lists: water 192 atoms 65, 66; 768: 95, 95; 1,536: 129, 124;
+// 3,072: 218, 209; 12,288: 470, 428; 512 structures of 157 atoms 3,140, 2,774;
+// crystal of 2,048 atoms (merged walk) 117, 109; 131,072: 2,960, 2,916; 30
+// functions of many eta, 768 atoms 105, 110; 1,536: 147, 144; 12,000: 549, 527.
+constexpr int kListAtoms = 1024;
+inline bool keep_lists(const Tuning& t, int natoms)
+{
+    return t.pair_lists == 1 || (t.pair_lists < 0 && natoms >= kListAtoms);
+}
 void setup_mixed(MixedModel& mm, const HostModel& hm);
 void update_mixed_weights(MixedModel& mm, const HostModel& hm);
 void free_mixed(MixedModel& mm);

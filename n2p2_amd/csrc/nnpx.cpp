@@ -112,6 +112,7 @@ struct nnpx_ctx {
     // setting the structures builds their list (it sizes the capacity): the
     // first evaluation of those positions takes that list
     bool list_fresh = false;
+    bool no_trips = false;       // no memory for pair lists that were not asked for
     bool settled = false;        // the flags of the work so far were read and clear
     // pinned host memory for small transfers (inputs; results and flags)
     DevBuf pin_in, pin_out;
@@ -934,11 +935,21 @@ MixedBuffers mixed_buffers(nnpx_ctx* c)
         m.keep.off = buf<int>(c, "keep_o", (size_t)c->N * (kMaxElem + 1));
     }
     const size_t tl = (size_t)c->N * c->trip_cap;
-    if (c->trip_cap > 0 && c->mixed.tune.pair_lists == 1 && !c->arena && tl * sizeof(unsigned) <= kTripBudget) {
-        m.trips.cap = c->trip_cap;
-        m.trips.ld = c->mixed.max_walks;
-        m.trips.list = buf<unsigned>(c, "trips", tl);
-        m.trips.counts = buf<int>(c, "trip_n", (size_t)c->N * kListWaves * m.trips.ld);
+    const bool asked = c->mixed.tune.pair_lists == 1;
+    if (c->trip_cap > 0 && keep_lists(c->mixed.tune, c->N) && !c->arena && tl * sizeof(unsigned) <= kTripBudget &&
+        (asked || !c->no_trips)) {
+        try {
+            m.trips.list = buf<unsigned>(c, "trips", tl);
+            m.trips.counts = buf<int>(c, "trip_n", (size_t)c->N * kListWaves * c->mixed.max_walks);
+            m.trips.cap = c->trip_cap;
+            m.trips.ld = c->mixed.max_walks;
+        } catch (const Fail&) {
+            // lists nobody asked for do not fail a call: evaluate without them
+            if (asked) throw;
+            (void)hipGetLastError();
+            m.trips = TripList{};
+            c->no_trips = true;
+        }
     }
     return m;
 }

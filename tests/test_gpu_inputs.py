@@ -111,6 +111,27 @@ def test_external_ragged(water, precision):
     same(result(m, precision), want, precision)
 
 
+@pytest.mark.parametrize("cells", [(6, 6, 9), (6, 7, 9)])
+def test_pair_lists_by_size(water, cells):
+    """972 and 1,134 atoms (no lists, lists from the second evaluation on): the
+    first evaluation, later ones, positions with more pairs than the lists were
+    sized for, and the lists switched off agree."""
+    say("case: pair lists by atom count,", 3 * int(np.prod(cells)), "atoms")
+    pos, elem, box = synth.water_box(9)
+    keep = np.all(np.indices((9, 9, 9)).reshape(3, -1).T < cells, axis=1)  # molecules in lattice order
+    pos, elem = pos.reshape(-1, 3, 3)[keep].reshape(-1, 3), elem.reshape(-1, 3)[keep].reshape(-1)
+    assert len(pos) == 3 * int(np.prod(cells))
+    box = np.diag(3.105 * np.array(cells, float))
+    m, off = n2p2_amd.Mode(water), n2p2_amd.Mode(water)
+    off.set_option(n2p2_amd.OPT_PAIR_LISTS, 0)
+    for f in (1.0, 0.93, 1.0):
+        m.set_structures(remap(f * pos, f * box), elem, (f * box)[None])
+        off.set_structures(remap(f * pos, f * box), elem, (f * box)[None])
+        want = result(off, n2p2_amd.MIXED)
+        for _ in range(3):
+            same(result(m, n2p2_amd.MIXED), want, n2p2_amd.MIXED)
+
+
 @pytest.mark.parametrize("precision", FORMS)
 def test_new_weights(water, precision):
     say("case: weights replaced and put back, precision", precision)
