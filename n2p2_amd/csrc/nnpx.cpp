@@ -2490,6 +2490,9 @@ namespace {
 void md_steps(nnpx_ctx* c, int nsteps, int graph_steps)
 {
     {
+        // the steps write the flags anew; a run that fails leaves them unread,
+        // and the next getter must then see them
+        c->settled = false;
         const bool timing = c->timing;
         if (graph_steps > 0 && (!c->gexec || c->graph_steps != graph_steps)) {
             drop_graph(c);
@@ -2530,7 +2533,6 @@ void md_steps(nnpx_ctx* c, int nsteps, int graph_steps)
         int f[4];
         read_flags(c, f);
         if (f[0] & 1) fail(NNPX_ERR_RANGE, "neighbour capacity exceeded during MD (raise the skin or re-initialise)");
-        c->settled = false;
         c->sf_valid = c->nn_valid = c->dedg_valid = c->e_valid = c->f_valid = true;
         c->sfd_valid = c->md_precision == NNPX_PLAIN_FP64 && !fused_fits(c);
         c->last_stored = c->sfd_valid;

@@ -179,3 +179,41 @@ def test_md_energy_conservation_and_rebuilds(fcc_dir):
     dF = float(np.abs(F - f.forces()).max())
     say("  final forces vs fresh evaluation: max|dF| %.2e" % dF)
     assert dF <= 1e-6
+
+
+@pytest.mark.parametrize("precision,graph_steps", [(n2p2_amd.MIXED, 0), (n2p2_amd.MIXED, 5), (n2p2_amd.PLAIN_FP64, 5)])
+def test_md_results_after_a_failed_run(fcc_dir, precision, graph_steps):
+    """A run that meets more neighbours than the list holds fails; the results
+    read after it are those of the positions it left, evaluated again with a
+    larger list, and not what the truncated one gave.  Two clusters of 216
+    atoms, one flying into the other: the first five steps fit (their results
+    are read, so the flags count as seen), the next five do not."""
+    say("case: MD, results after a run past the list capacity, precision %d, graph steps %d" % (precision, graph_steps))
+    g = 1.8 * np.arange(6)
+    one = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    one = one + np.random.default_rng(91).normal(0.0, 0.05, one.shape)
+    pos = np.concatenate([one, one + [60.0, 0.9, 0.9]])
+    elem = (np.arange(len(pos)) % 4).astype(np.int32)
+    vel = np.zeros_like(pos)
+    vel[len(one):, 0] = -(60.0 - 0.9) / 10
+    m = n2p2_amd.Mode(fcc_dir)
+    m.set_option(n2p2_amd.OPT_MD_STAGING, 0)
+    m.set_structures(pos, elem)
+    m.md_init(np.full(4, 1e6), vel, 1.0, 0.0, precision)
+    m.md_run(5, graph_steps=graph_steps)
+    m.energies()
+    with pytest.raises(n2p2_amd.NNPError, match="capacity exceeded"):
+        m.md_run(5, graph_steps=graph_steps)
+    E, F = m.energies()[0], m.forces()
+    x, _ = m.md_state()
+    f = n2p2_amd.Mode(fcc_dir)
+    f.set_structures(x, elem)
+    f.evaluate(precision, forces=True)
+    E0, F0 = f.energies()[0], f.forces()
+    top = float(np.abs(F0).max())
+    say("  rel dE %.2e  max|dF| %.2e of %.2e" % (abs(E - E0) / abs(E0), float(np.abs(F - F0).max()), top))
+    # the same kernels on the same positions: FP64 sums in another order, and
+    # in the mixed form FP32 sums in another order (6e-8 a rounding, up to a
+    # hundred terms)
+    tol = 1e-12 if precision == n2p2_amd.PLAIN_FP64 else 1e-5
+    assert abs(E - E0) <= tol * abs(E0) and np.abs(F - F0).max() <= tol * top
