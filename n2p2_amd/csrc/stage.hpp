@@ -8,7 +8,10 @@
 
 namespace nnpx {
 
-constexpr int kStagePasses = 16;  // 64-entry passes of the longest list (1,024 entries)
+// 64-entry passes of a list with counts of their own (1,024 entries).  A longer
+// list (MD lists with a skin: the limit is checked where a list is fitted, and a
+// fitted capacity leaves room for more) has the rest of its passes in the last one.
+constexpr int kStagePasses = 16;
 
 // Lane of the wave, and the wave's number in the block as a scalar.
 __device__ inline int lane_id() { return threadIdx.x & (kWave - 1); }
@@ -19,8 +22,9 @@ __device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane(threadId
 // them) in slots grouped by neighbour element and in list order within an
 // element, so element e's neighbours are the slots eoff[e] .. eoff[e + 1] - 1:
 // store(slot, entry, vector, distance, element) for each.  The block's wave w
-// (of W) takes the list's 64-entry passes w, w + W, ...; cnt is LDS for
-// kStagePasses * kMaxElem counts.  More such entries than capL: only slots
+// (of W) takes the list's 64-entry passes w, w + W, ..., and the one with the
+// last of kStagePasses all that follow it; cnt is LDS for kStagePasses *
+// kMaxElem counts.  More such entries than capL: only slots
 // below capL are stored, flag bit 4 is set (the caller repeats with the full
 // capacity) and flags[2] keeps the largest count met.  Returns the slots in
 // use; starts and ends with the block in step.
@@ -32,7 +36,9 @@ __device__ inline int stage_by_element(const ModelT* __restrict__ M, const SysVi
     const StructT& St = s.st[s.sid[i]];
     const int nl = s.nb_n[i];
     const int ne = M->nelem;
-    const int npass = min((nl + kWave - 1) / kWave, kStagePasses);
+    constexpr int kLast = kStagePasses - 1;
+    const int passes = (nl + kWave - 1) / kWave, npass = min(passes, kStagePasses);
+    const int mine = kLast % W == wv ? passes : npass;  // end of this wave's passes
     const size_t base = (size_t)i * s.cap;
     const double rmax = M->maxCutoff;
     struct Entry {
@@ -56,7 +62,10 @@ __device__ inline int stage_by_element(const ModelT* __restrict__ M, const SysVi
     auto count = [&](int p, int el) {
         for (int e = 0; e < ne; ++e) {
             const int c = __popcll(__ballot(el == e));
-            if (lane == 0) cnt[p * kMaxElem + e] = c;
+            if (lane == 0) {
+                int& row = cnt[min(p, kLast) * kMaxElem + e];
+                row = p > kLast ? row + c : c;
+            }
         }
     };
 #pragma unroll
@@ -68,7 +77,7 @@ __device__ inline int stage_by_element(const ModelT* __restrict__ M, const SysVi
             count(p, keep[q].el);
         }
     }
-    for (int p = wv + kKeep * W; p < npass; p += W) count(p, entry(p).el);
+    for (int p = wv + kKeep * W; p < mine; p += p < kLast ? W : 1) count(p, entry(p).el);
     __syncthreads();
     // lane e: element e's entries, its first slot, and the next of this wave's pass
     int tot = 0;
@@ -79,7 +88,7 @@ __device__ inline int stage_by_element(const ModelT* __restrict__ M, const SysVi
     int next = incl - tot, seen = 0;
     if (wv == 0 && lane <= ne) eoff[lane] = min(lane < ne ? next : total, capL);
     auto place = [&](int p, const Entry& x) {
-        for (; seen < p; ++seen)
+        for (; seen < min(p, kLast); ++seen)
             if (lane < ne) next += cnt[seen * kMaxElem + lane];
         int pos = -1;
         for (int e = 0; e < ne; ++e) {
@@ -88,13 +97,14 @@ __device__ inline int stage_by_element(const ModelT* __restrict__ M, const SysVi
             if (x.el == e)
                 pos = at + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                           __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            if (p >= kLast && lane == e) next += __popcll(m);  // for the passes that share its row
         }
         if (pos >= 0 && pos < capL) store(pos, p * kWave + lane, x.dr, x.d, x.el);
     };
 #pragma unroll
     for (int q = 0; q < kKeep; ++q)
         if (wv + q * W < npass) place(wv + q * W, keep[q]);
-    for (int p = wv + kKeep * W; p < npass; p += W) place(p, entry(p));
+    for (int p = wv + kKeep * W; p < mine; p += p < kLast ? W : 1) place(p, entry(p));
     if (threadIdx.x == 0) {
         if (total > capL) atomicOr(&s.flags[0], 4);
         if (total > __hip_atomic_load(&s.flags[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))

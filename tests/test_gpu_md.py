@@ -217,3 +217,36 @@ def test_md_results_after_a_failed_run(fcc_dir, precision, graph_steps):
     # hundred terms)
     tol = 1e-12 if precision == n2p2_amd.PLAIN_FP64 else 1e-5
     assert abs(E - E0) <= tol * abs(E0) and np.abs(F - F0).max() <= tol * top
+
+
+def test_md_list_past_1024_entries(fcc_dir):
+    """A list of more than 1,024 entries, few of them inside the cutoff, as an
+    MD list with a skin may grow to: every entry is staged.  980 atoms, and 120
+    far from them when the list is sized and near them when it is evaluated;
+    the entries past 1,024 are neighbours of the 120."""
+    say("case: MD list of 1,099 entries, mixed form")
+    g = 2.4 * np.arange(10)
+    grid = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    rng = np.random.default_rng(92)
+    pos = np.concatenate([grid[:980], grid[:120] + [40.0, 0.0, 0.0]]) + rng.normal(0.0, 0.05, (1100, 3))
+    elem = rng.integers(0, 4, len(pos)).astype(np.int32)
+    apart = pos.copy()
+    apart[980:, 0] += 260.0
+    m = n2p2_amd.Mode(fcc_dir)
+    m.set_structures(apart, elem)
+    m.md_init(masses_fcc(), np.zeros_like(pos), 1.0, 100.0, n2p2_amd.MIXED)
+    m.update_positions(pos)
+    f = n2p2_amd.Mode(fcc_dir)
+    f.set_structures(pos, elem)
+    rng = np.random.default_rng(93)
+    vE, vF = rng.normal(size=1), rng.normal(size=pos.shape)
+    got = []
+    for x in (m, f):
+        x.evaluate(n2p2_amd.MIXED, forces=True)
+        got.append([x.G(), x.energies(), x.forces(), x.weight_vjp(vE, vF, n2p2_amd.MIXED)])
+    assert m.neighbors()[0].max() == len(pos) - 1
+    # equal terms; FP32 sums of up to a hundred of them in another order
+    for what, a, b in zip(("G", "energy", "forces", "rows"), *got):
+        err = float(np.abs(a - b).max() / np.abs(b).max())
+        say("  %s: max rel %.2e" % (what, err))
+        assert err <= 1e-5
