@@ -669,8 +669,22 @@ inline void dispatch_angular(const MixedModel& mm, const ModelT& t, int maxm, F&
 // Crystal of 256 atoms (merged walk) 91, 69, 61; 2,048: 128, 117, 132; 6,912:
 // 268, 260, 320.  30 functions of many eta (member path): 192 atoms 153, 96, 71;
 // 1,536: 181, 147, 150.
+// Fewer where the staging with the smallest buffers does not fit beside them
+// (from 961 slots on), for all kernels alike: the SF and the force kernel share
+// pair lists per wave.
 constexpr int kFewAtoms = 1024, kSomeAtoms = 4096;
-inline int waves_per_atom(int natoms) { return natoms <= kFewAtoms ? 4 : natoms <= kSomeAtoms ? 2 : 1; }
+inline int waves_per_atom(const MixedModel& mm, const SysView& s)
+{
+    const int nbas = 2 * (mm.powNB[0] + mm.powNB[1]);
+    auto fits = [&](int w) {
+        const size_t st = stage_bytes(s.stage_cap, w, kWave, stage_mp(mm.powNB[0], mm.powNB[1], w));
+        return st + merge_bytes(mm.merge_ng, nbas, w) <= 65536 &&
+               st + merge_bytes(mm.merge_ng, nbas, 1) + (sizeof(double) * 3 + 2) * (size_t)s.stage_cap <= 65536;
+    };
+    int w = s.natoms <= kFewAtoms ? 4 : s.natoms <= kSomeAtoms ? 2 : 1;
+    while (w > 1 && !fits(w)) w /= 2;
+    return w;
+}
 
 // Entries of each wave's triplet buffer: the tuned size, less where the
 // staging of capL neighbours (fixed bytes beside the buffers) leaves no room.

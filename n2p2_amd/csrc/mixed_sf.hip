@@ -508,7 +508,7 @@ void launch_sf32(const MixedModel& mm, const ModelT& t, const ModelT* d_model, c
     const int capL = s.stage_cap;
     const int P = pow2_members(t);
     const int tsf = mm.tune.trip_sf;
-    dispatch_waves(waves_per_atom(s.natoms), [&](auto wc) {
+    dispatch_waves(waves_per_atom(mm, s), [&](auto wc) {
           dispatch_angular(mm, t, P, [&](auto m, auto fast, auto nb0, auto nb1, auto cs) {
             constexpr int W = decltype(wc)::value;
             constexpr int cm = decltype(m)::value, c0 = decltype(nb0)::value, c1 = decltype(nb1)::value;

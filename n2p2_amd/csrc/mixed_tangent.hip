@@ -265,14 +265,16 @@ void launch_tangent32(const MixedModel& mm, const ModelT& t, const ModelT* d_mod
     const size_t extra = (sizeof(float4) + 2) * (size_t)capL;
     if (stage_bytes(capL, 1, tt, stage_mp(0, 0, 1)) + extra > 65536)
         throw Error{NNPX_ERR_UNSUPPORTED, "neighbour count too large for the mixed kernels' LDS"};
-    if (t.has_exp) dispatch_waves(waves_per_atom(s.natoms), [&](auto wc) {
+    if (t.has_exp) dispatch_waves(waves_per_atom(mm, s), [&](auto wc) {
         dispatch_angular(mm, t, pow2_members(t), [&](auto m, auto fast, auto nb0, auto nb1, auto cs) {
             constexpr int W = decltype(wc)::value, c0 = decltype(nb0)::value, c1 = decltype(nb1)::value;
             constexpr int mp = stage_mp(c0, c1, W);
             const int trip = wave_trip(tt, W, stage_bytes(capL, 0, 0, mp) + extra);
+            const size_t lds = stage_bytes(capL, W, trip, mp) + extra;
+            if (lds > 65536) throw Error{NNPX_ERR_UNSUPPORTED, "neighbour count too large for the mixed kernels' LDS"};
             hipLaunchKernelGGL((k_tangent32<W, decltype(m)::value, decltype(fast)::value, c0, c1, decltype(cs)::value>),
-                               dim3(s.natoms), dim3(W * kWave), stage_bytes(capL, W, trip, mp) + extra, stream, d_model,
-                               mm.d_mem, mm.d_gmix, s, u, mm.d_sffac, Gdot, ldG, capL, trip);
+                               dim3(s.natoms), dim3(W * kWave), lds, stream, d_model, mm.d_mem, mm.d_gmix, s, u,
+                               mm.d_sffac, Gdot, ldG, capL, trip);
         });
     });
     launch_tangentcomp32(d_model, t, s, u, Gdot, ldG, stream);

@@ -565,3 +565,61 @@ def test_pair_lists(kind, water_dir, tmp_path):
     rms, mx, erel = errors(m, o)
     say("  lists off: E rel %.2e  F rms %.2e max %.2e" % (erel, rms, mx))
     assert erel <= 1e-5 and rms <= 1e-5
+
+
+def test_few_atoms_with_the_longest_lists(tmp_path):
+    """975 atoms with up to 974 neighbours each, member-path functions: the
+    staging leaves no room for the buffers of the four waves that this few
+    atoms take otherwise.  Against the plain form's functions, and against the
+    same atoms among 3,200 others (one wave each)."""
+    say("case: 975 atoms in a ball of 974 neighbours, mixed")
+    lines = []
+    for c in ("H", "O"):
+        lines += ["%s 2 %s 0.05 0.0 6.35" % (c, n) for n in "HO"]
+        for a, b in (("H", "H"), ("H", "O"), ("O", "O")):
+            lines += ["%s 3 %s %s 0.02 %.1f %.1f 6.35" % (c, a, b, lam, zeta) for lam in (1.0, -1.0) for zeta in (1.0, 3.0)]
+    d = str(tmp_path / "members")
+    sfs = synth.sorted_sfs(lines, ("H", "O"))
+    rows = [(e + 1, k + 1, 0.0, 1.0, 0.0, 1.0) for e in range(2) for k in range(len(sfs[e]))]
+
+    def ball(n):
+        g = 0.97 * np.arange(-8, 9)
+        p = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+        p = p[np.argsort((p * p).sum(1), kind="stable")[:n]]
+        return p + np.random.default_rng(61).normal(0.0, 0.03, p.shape)
+    pos = ball(975)
+    elem = (np.arange(975) % 3 == 0).astype(np.int32)
+    # the networks see the functions' own ranges
+    synth.write_model(d, ("H", "O"), lines, (10, 10), ("t", "t", "l"), rows, scaling=False)
+    m = n2p2_amd.Mode(d)
+    m.set_structures(pos, elem)
+    m.evaluate(n2p2_amd.PLAIN_FP64, forces=False)
+    G = m.G()
+    rows = [(e + 1, k + 1, 0.0, 2.0 * G[elem == e, k].max(), 0.0, 1.0) for e in range(2) for k in range(len(sfs[e]))]
+    synth.write_model(d, ("H", "O"), lines, (10, 10), ("t", "t", "l"), rows)
+    m = n2p2_amd.Mode(d)
+    m.set_structures(pos, elem)
+    assert m.neighbors()[0].max() > 960
+    m.evaluate(n2p2_amd.PLAIN_FP64, forces=False)
+    G, E = m.G(), m.energies()[0]
+    m.evaluate(n2p2_amd.MIXED, forces=True)
+    gerr = float(np.abs(m.G() - G).max() / np.abs(G).max())
+    eerr = abs(m.energies()[0] - E) / abs(E)
+    F = m.forces()
+    rng = np.random.default_rng(62)
+    vE, vF = rng.normal(size=1), rng.normal(size=pos.shape)
+    row = m.weight_vjp(vE, vF, n2p2_amd.MIXED)
+    far = 50.0 * np.stack(np.meshgrid(*[np.arange(1, 18)] * 3, indexing="ij"), -1).reshape(-1, 3)[:3200]
+    m.set_structures(np.concatenate([pos, far]), np.concatenate([elem, np.zeros(3200, np.int32)]),
+                     None, [0, 975, 4175])
+    m.evaluate(n2p2_amd.MIXED, forces=True)
+    F1 = m.forces()[:975]
+    row1 = m.weight_vjp(np.append(vE, 0.0), np.concatenate([vF, np.zeros((3200, 3))]), n2p2_amd.MIXED)
+    ferr = float(np.abs(F - F1).max() / np.abs(F1).max())
+    rerr = float(np.abs(row - row1[:1]).max() / np.abs(row).max())
+    say("  G rel %.2e  E rel %.2e  forces %.2e  rows %.2e" % (gerr, eerr, ferr, rerr))
+    # FP32 terms and compensated sums; two bf16 parts of an operand (1.5e-5)
+    # through four products; the same terms in another order, sums of some
+    # thousand of them per lane in the forces and compensated ones in the rows
+    assert gerr <= 2e-6 and eerr <= 1e-4
+    assert ferr <= 5e-5 and rerr <= 2e-5
