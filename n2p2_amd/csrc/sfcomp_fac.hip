@@ -29,9 +29,10 @@
 //   Bound by instruction issue at two or three waves per SIMD (294 vector
 // instructions per triplet for 54 values, 480 for their forces; 64 FP64 sums
 // take 128 registers).  184 functions and 185 neighbours per atom, 1,152 atoms,
-// FP32 terms: values 4,344 us member by member -> 340 us, forces 4,872 -> 383
+// FP32 terms: values 4,344 us member by member -> 335 us, forces 4,872 -> 377
 // us (647 and 639 with a switch over the cores and a window test per function
-// in the walk).
+// in the walk; forces 370 with a run's sums in FP32, which cost up to 8e-7 of a
+// sum of 392 like terms, against 1.8e-7 for the terms alone).
 #include <type_traits>
 
 #include "nnpx.h"
@@ -287,17 +288,17 @@ __global__ __launch_bounds__(kFT) void k_sfcomp_fac(const ModelT* __restrict__ M
         int cur = -1;
         V4 gj{};
         T rij = T(0), Rj[RW], dRj[DER ? RW : 1];
-        T sx = T(0), sy = T(0), sz = T(0), hx = T(0), hy = T(0), hz = T(0);
+        double sx = 0.0, sy = 0.0, sz = 0.0, hx = 0.0, hy = 0.0, hz = 0.0;  // sums of a run of one j
         T wjx = T(0), wjy = T(0), wjz = T(0);
         auto flush = [&] {
             if constexpr (FORCE) {
                 if (cur >= 0) {
-                    lds_add(ax + cur, (double)hx);
-                    lds_add(ax + capL + cur, (double)hy);
-                    lds_add(ax + 2 * capL + cur, (double)hz);
-                    fx -= (double)sx;
-                    fy -= (double)sy;
-                    fz -= (double)sz;
+                    lds_add(ax + cur, hx);
+                    lds_add(ax + capL + cur, hy);
+                    lds_add(ax + 2 * capL + cur, hz);
+                    fx -= sx;
+                    fy -= sy;
+                    fz -= sz;
                 }
             }
         };
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(kFT) void k_sfcomp_fac(const ModelT* __restrict__ M
                 rij = ri[j];
                 load_row(R + j * RW, Rj);
                 if constexpr (DER) load_row(dR + j * RW, dRj);
-                sx = sy = sz = hx = hy = hz = T(0);
+                sx = sy = sz = hx = hy = hz = 0.0;
                 if (TANGENT) {
                     wjx = (T)ax[j];
                     wjy = (T)ax[capL + j];
@@ -389,12 +390,12 @@ __global__ __launch_bounds__(kFT) void k_sfcomp_fac(const ModelT* __restrict__ M
                 const T P1 = rij * (rik - rij * cost) * X + rij * Y1;
                 const T P2 = rik * (rij - rik * cost) * X + rik * Y2;
                 const T d1 = P1 - P3, d2 = P2 - P3;
-                sx += P1 * gj.x + P2 * gk.x;
-                sy += P1 * gj.y + P2 * gk.y;
-                sz += P1 * gj.z + P2 * gk.z;
-                hx += d1 * gj.x + P3 * gk.x;
-                hy += d1 * gj.y + P3 * gk.y;
-                hz += d1 * gj.z + P3 * gk.z;
+                sx += (double)(P1 * gj.x + P2 * gk.x);
+                sy += (double)(P1 * gj.y + P2 * gk.y);
+                sz += (double)(P1 * gj.z + P2 * gk.z);
+                hx += (double)(d1 * gj.x + P3 * gk.x);
+                hy += (double)(d1 * gj.y + P3 * gk.y);
+                hz += (double)(d1 * gj.z + P3 * gk.z);
                 lds_add(ax + k, (double)(d2 * gk.x + P3 * gj.x));
                 lds_add(ax + capL + k, (double)(d2 * gk.y + P3 * gj.y));
                 lds_add(ax + 2 * capL + k, (double)(d2 * gk.z + P3 * gj.z));

@@ -87,3 +87,36 @@ def test_factored_against_members(kind, atoms, tmp_path):
             err = float(np.abs(a - b).max() / max(np.abs(b).max(), 1e-300)) if np.abs(b).max() > 0 else np.abs(a).max()
             say("  %s %s %s %s: max rel %.2e" % (kind, atoms, name, what, err))
             assert np.isfinite(a).all() and err <= t
+
+
+def test_force_sums_in_64_bits(tmp_path):
+    """The mixed form's compact forces have FP32 terms and FP64 sums.  One atom
+    with functions, eight neighbours on an axis and 392 on a ring around it, at
+    right angles, where the angular function is at its maximum: along the axis
+    the force on one of the eight is a sum of 392 terms that are equal up to
+    rounding.  FP32 sums would round the same way each time, by up to half an
+    ulp of the sum: 5e-7 and more.  The terms' errors, which all share, are
+    some four roundings of 6e-8, one of them tripled by the polynomial's
+    cancellation: 3e-7 at the most.  The linear network's weights
+    (powers of two) are exact in both forms."""
+    say("case: compact force sums, 400 neighbours, mixed against plain")
+    lines = ["O 22 H H %g %g 0.0 180.0 p2" % (-r, r) for r in (5.0, 5.5, 6.0)]
+    lines += ["H 20 O 0.0 0.3 p2"]
+    sfs = synth.sorted_sfs(lines, ("H", "O"))
+    rows = [(e + 1, k + 1, 0.0, 1.0, 0.0, 1.0) for e in range(2) for k in range(len(sfs[e]))]
+    weights = {c: np.concatenate([np.full(n, 0.25), [0.0], [1.0], [0.0]]) for c, n in (("H", 1), ("O", 3))}
+    d = str(tmp_path / "star")
+    synth.write_model(d, ("H", "O"), lines, (1,), ("l", "l"), rows, weights=weights)
+    phi = np.arange(392) * (2.0 * np.pi / 392)
+    ring = 2.5 * np.stack([np.cos(phi), np.sin(phi), np.zeros(392)], 1)
+    pos = np.concatenate([np.zeros((1, 3)), [[0.0, 0.0, 0.6 + 0.19 * k] for k in range(8)], ring])
+    elem = np.array([1] + [0] * 400, np.int32)
+    F = {}
+    for precision in (n2p2_amd.PLAIN_FP64, n2p2_amd.MIXED):
+        m = n2p2_amd.Mode(d)
+        m.set_structures(pos, elem)
+        m.evaluate(precision, forces=True)
+        F[precision] = m.forces()[1:9, 2]
+    err = np.abs(F[n2p2_amd.MIXED] / F[n2p2_amd.PLAIN_FP64] - 1.0)
+    say("  rel errors", " ".join("%.1e" % x for x in err))
+    assert err.max() <= 3e-7
