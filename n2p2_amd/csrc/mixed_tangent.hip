@@ -15,10 +15,11 @@ namespace {
 // scaled like the SFs themselves (scaling factor and angular normalisation).
 // Power path (NB0 > 0): per triplet one exponential per eta and the powers of
 // the two bases, a term's tangent being E (p^(2^b) x + 2^b p^(2^b - 1) y) with
-// x, y shared by the terms; terms summed over a buffer in FP32, then folded
-// into compensated sums, as the values are.  Bound by instruction issue like
-// the force kernel; 41,000 atoms, 30 angular functions per element: 1,342 us
-// with an exponential per member, 939 us so.
+// x, y shared by the terms; FP64 sums per lane (the terms have both signs; a
+// conversion and an addition, less than compensation).  Bound by instruction
+// issue like the force kernel; 41,000 atoms, 30 angular functions per element:
+// 1,342 us with an exponential per member, 972 us so (932 with FP32 sums over
+// a buffer, which differ by up to 2e-7 with its size).
 template <int W, int MAXM, bool FAST, int NB0, int NB1, bool COS>
 __global__ __launch_bounds__(W * kWave) void k_tangent32(const ModelT* __restrict__ M, const MemberF* __restrict__ MF,
                                                          const GroupMixF* __restrict__ GM, SysView s,
@@ -101,11 +102,15 @@ __global__ __launch_bounds__(W * kWave) void k_tangent32(const ModelT* __restric
         constexpr int NBAS = POW ? 2 * (NB0 + NB1) : 1;
         constexpr int NBM = NB0 > NB1 ? NB0 : NB1;
         constexpr int NACC = POW ? NBAS : MAXM;
-        float acc[NACC], cmp[NACC], part[NBAS];
+        // sums of terms of both signs: FP64, or FP32 with compensation per member
+        using Sum = std::conditional_t<POW, double, float>;
+        Sum acc[NACC];
+        float cmp[POW ? 1 : MAXM];
 #pragma unroll
-        for (int q = 0; q < NACC; ++q) { acc[q] = 0.f; cmp[q] = 0.f; }
-#pragma unroll
-        for (int q = 0; q < NBAS; ++q) part[q] = 0.f;
+        for (int q = 0; q < NACC; ++q) {
+            acc[q] = 0;
+            if (!POW) cmp[q] = 0.f;
+        }
         const bool same = GT.e1 == GT.e2;
         const bool wide = GT.type == 9;  // no r_jk cutoff or exponent term (SymGrpExpAngw.cpp:156-380)
         const bool wt = GT.type == 13;    // Z_j Z_k weights (SymGrpExpAngnWeighted.cpp)
@@ -159,11 +164,8 @@ __global__ __launch_bounds__(W * kWave) void k_tangent32(const ModelT* __restric
                     float y0 = E0 * al * gm.lam[sl], y1 = E1 * al * gm.lam[sl];  // times zeta = 2^b
 #pragma unroll
                     for (int b = 0; b < NBM; ++b) {
-                        if (b < NB0) part[sl * NB0 + b] = fmaf(x0, p, fmaf(y0, pq, part[sl * NB0 + b]));
-                        if (b < NB1) {
-                            const int t = 2 * NB0 + sl * NB1 + b;
-                            part[t] = fmaf(x1, p, fmaf(y1, pq, part[t]));
-                        }
+                        if (b < NB0) acc[sl * NB0 + b] += (double)fmaf(x0, p, y0 * pq);
+                        if (b < NB1) acc[2 * NB0 + sl * NB1 + b] += (double)fmaf(x1, p, y1 * pq);
                         pq *= p;
                         p *= p;
                         y0 += y0;
@@ -223,14 +225,6 @@ __global__ __launch_bounds__(W * kWave) void k_tangent32(const ModelT* __restric
                         }
                 }
             }
-        }, [&]() {
-            if constexpr (POW) {
-#pragma unroll
-                for (int b = 0; b < NBAS; ++b) {
-                    kahan(acc[b], cmp[b], part[b]);
-                    part[b] = 0.f;
-                }
-            }
         });
         // the waves' sums pass through their own buffers
         double* red = reinterpret_cast<double*>(S.tjk);
@@ -238,7 +232,9 @@ __global__ __launch_bounds__(W * kWave) void k_tangent32(const ModelT* __restric
 #pragma unroll
         for (int q = 0; q < NACC; ++q)
             if (POW || q < nmem) {
-                const double v = wave_sum((double)acc[q] + (double)cmp[q]);
+                double v = (double)acc[q];
+                if constexpr (!POW) v += (double)cmp[q];
+                v = wave_sum(v);
                 if (lane == 0) red[q] = v;
             }
         __syncthreads();

@@ -290,3 +290,43 @@ def test_gradient_tiles(models, precision, per_block):
     relg = float(np.abs(g - n * g0).max() / np.abs(n * g0).max())
     say("  rows max rel %.2e, summed gradient max rel %.2e" % (rel, relg))
     assert max(rel, relg) <= (1e-12 if precision == n2p2_amd.PLAIN_FP64 else 1e-5)
+
+
+def test_tangent_sums_in_64_bits(tmp_path):
+    """The mixed form's tangent has FP32 terms; the buffer of pairs that a lane
+    sums before it folds them must not show.  One atom with functions, eight
+    neighbours as good as in one place and 392 on a ring around their axis: with
+    a field on the eight, a lane's buffer is tens of equal terms, whose FP32 sum
+    would round the same way each time.  A linear network with weights that are
+    powers of two, no seed on the energy: a row is the functions' tangents."""
+    say("case: tangent, 400 neighbours, buffers of 64 and 4,096 pairs")
+    lines = ["O 9 H H 0.01 %.1f %.1f 6.0" % (lam, zeta) for lam in (1.0, -1.0) for zeta in (1.0, 2.0, 4.0)]
+    lines += ["O 9 H H 0.04 1.0 1.0 6.0", "H 2 O 0.05 0.0 0.3"]
+    sfs = synth.sorted_sfs(lines, ("H", "O"))
+    rows = [(e + 1, k + 1, 0.0, 1.0, 0.0, 1.0) for e in range(2) for k in range(len(sfs[e]))]
+    weights = {c: np.concatenate([np.full(n, 0.25), [0.0], [1.0], [0.0]]) for c, n in (("H", 1), ("O", 7))}
+    d = str(tmp_path / "star")
+    synth.write_model(d, ("H", "O"), lines, (1,), ("l", "l"), rows, weights=weights)
+    phi = np.arange(392) * (2.0 * np.pi / 392)
+    ring = 2.5 * np.stack([np.cos(phi), np.sin(phi), np.zeros(392)], 1)
+    worst = [0.0, 0.0]
+    for z in (0.9, 1.3, 1.7, 2.3):
+        pos = np.concatenate([np.zeros((1, 3)), [[0.0, 0.0, z + 1e-7 * k] for k in range(8)], ring])
+        elem = np.array([1] + [0] * 400, np.int32)
+        u = np.zeros_like(pos)
+        u[1:9, 2] = 1.0
+        m = n2p2_amd.Mode(d)
+        m.set_structures(pos, elem)
+        t = m.tuning()
+        got = {}
+        for trip in (64, 4096):
+            m.set_tuning(t["trip_sf"], t["trip_force"], trip, t["grad_atoms"])
+            got[trip] = m.weight_vjp(np.zeros(1), u, n2p2_amd.MIXED)[0]
+        plain = m.weight_vjp(np.zeros(1), u, n2p2_amd.PLAIN_FP64)[0]
+        k = np.abs(plain) > 1e-3 * np.abs(plain).max()
+        for q, (a, b) in enumerate(((got[4096], got[64]), (got[64], plain))):
+            worst[q] = max(worst[q], float(np.abs(a[k] / b[k] - 1.0).max()))
+    say("  large against small buffers %.1e, against the plain form %.1e" % tuple(worst))
+    # the network pass takes the tangent rounded to FP32 (6e-8 each side); a
+    # term has a dozen FP32 factors, two of them hardware sines and cosines
+    assert worst[0] <= 1.2e-7 and worst[1] <= 2e-6
