@@ -112,7 +112,7 @@ struct nnpx_ctx {
     // setting the structures builds their list (it sizes the capacity): the
     // first evaluation of those positions takes that list
     bool list_fresh = false;
-    bool no_trips = false;       // no memory for pair lists that were not asked for
+    size_t no_trips = 0;         // bytes of pair lists, not asked for, that could not be had (0: none)
     bool settled = false;        // the flags of the work so far were read and clear
     // pinned host memory for small transfers (inputs; results and flags)
     DevBuf pin_in, pin_out;
@@ -936,8 +936,9 @@ MixedBuffers mixed_buffers(nnpx_ctx* c)
     }
     const size_t tl = (size_t)c->N * c->trip_cap;
     const bool asked = c->mixed.tune.pair_lists == 1;
-    if (c->trip_cap > 0 && keep_lists(c->mixed.tune, c->N) && !c->arena && tl * sizeof(unsigned) <= kTripBudget &&
-        (asked || !c->no_trips)) {
+    const size_t tb = tl * sizeof(unsigned);
+    if (c->trip_cap > 0 && keep_lists(c->mixed.tune, c->N) && !c->arena && tb <= kTripBudget &&
+        (asked || c->no_trips == 0 || tb < c->no_trips)) {
         try {
             m.trips.list = buf<unsigned>(c, "trips", tl);
             m.trips.counts = buf<int>(c, "trip_n", (size_t)c->N * kListWaves * c->mixed.max_walks);
@@ -945,10 +946,16 @@ MixedBuffers mixed_buffers(nnpx_ctx* c)
             m.trips.ld = c->mixed.max_walks;
         } catch (const Fail&) {
             // lists nobody asked for do not fail a call: evaluate without them
+            // (smaller ones, and another model's, are tried again)
             if (asked) throw;
             (void)hipGetLastError();
             m.trips = TripList{};
-            c->no_trips = true;
+            c->no_trips = tb;
+            for (const char* name : {"trips", "trip_n"}) {  // what was had of them
+                DevBuf& b = c->bufs[name];
+                if (b.p) (void)hipFree(b.p);
+                b = DevBuf{};
+            }
         }
     }
     return m;
@@ -1132,6 +1139,7 @@ nnpx_status nnpx_load_model(nnpx_ctx* c, const char* dir)
         double* dfac = buf<double>(c, "fac64", fac.size());
         hip_check(hipMemcpy(dfac, fac.data(), sizeof(double) * fac.size(), hipMemcpyHostToDevice), "hipMemcpy");
         c->has_model = true;
+        c->no_trips = 0;
         c->N = c->S = 0;
         c->nbr_valid = false;
         invalidate(c);
