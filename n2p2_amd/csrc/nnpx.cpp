@@ -2504,6 +2504,9 @@ void md_steps(nnpx_ctx* c, int nsteps, int graph_steps)
         const bool timing = c->timing;
         if (graph_steps > 0 && (!c->gexec || c->graph_steps != graph_steps)) {
             drop_graph(c);
+            // nothing can be allocated under capture: the pair lists may have
+            // been turned on since the set-up
+            if (c->md_precision == NNPX_MIXED) (void)mixed_buffers(c);
             c->timing = false;  // no event records inside the captured sequence
             hip_check(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
             try {

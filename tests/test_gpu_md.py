@@ -250,3 +250,26 @@ def test_md_list_past_1024_entries(fcc_dir):
         err = float(np.abs(a - b).max() / np.abs(b).max())
         say("  %s: max rel %.2e" % (what, err))
         assert err <= 1e-5
+
+
+def test_md_graph_after_pair_list_option(fcc_dir):
+    """Pair lists left to the library again after nnpx_md_init ran without
+    them: the lists are there before the steps are captured."""
+    say("case: MD graph, pair lists 0 at init, -1 at the run, FCC 2,048")
+    pos, elem, box = synth.fcc_lattice(n_cells=8)
+    mass = masses_fcc()
+    vel = synth.maxwell_velocities(mass[elem], 600.0, synth.SEED_VELOCITY)
+    got = []
+    for graph_steps in (5, 0):
+        m = n2p2_amd.Mode(fcc_dir)
+        m.set_structures(remap(pos, box), elem, box[None])
+        m.evaluate(n2p2_amd.MIXED, forces=True)
+        m.energies()  # the lists' size is known from here on, and no list kept yet
+        m.set_option(n2p2_amd.OPT_PAIR_LISTS, 0)
+        m.md_init(mass, vel, 1.0, 0.5, n2p2_amd.MIXED)
+        m.set_option(n2p2_amd.OPT_PAIR_LISTS, -1)
+        m.md_run(10, graph_steps=graph_steps)
+        got.append(m.md_state()[0])
+    dx = float(np.abs(got[0] - got[1]).max())
+    say("  graph vs eager max|dx| %.2e" % dx)
+    assert dx <= 1e-9
