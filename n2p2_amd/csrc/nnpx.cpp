@@ -1381,7 +1381,7 @@ nnpx_status nnpx_calculate_symmetry_function_groups(nnpx_ctx* c, int derivatives
         need_structures(c);
         if (!c->nbr_valid) build_neighbors(c, true);
         // Mode.cpp:1634-1635: skip when results are already there
-        if (stored_dgdr(c) || (c->sf_valid && !derivatives)) return;
+        if ((c->sf_valid && !derivatives) || stored_dgdr(c)) return;
         compute_sf64(c, derivatives != 0);
         c->nn_valid = c->dedg_valid = c->e_valid = c->f_valid = false;
     });

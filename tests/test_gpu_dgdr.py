@@ -198,3 +198,25 @@ def test_facade_copies_dGdr(tmp_path):
         p += counts[i]
     say("  max rel err %.2e over %d atoms, %d entries" % (worst, len(atoms), p))
     assert worst <= TOL
+
+
+def test_dGdr_after_a_gradient_on_demand(tmp_path):
+    """A plain gradient leaves dG/dr to be had, and it is computed and stored
+    by the call that asks for it and by no other."""
+    d = synth.water_model(str(tmp_path / "water"))
+    pos, elem, box = synth.water_box(2)
+    m = n2p2_amd.Mode(d)
+    m.set_structures(pos, elem, box[None])
+    m.weight_vjp(np.ones(1), np.ones_like(pos), n2p2_amd.PLAIN_FP64)
+    m.set_option(n2p2_amd.OPT_TIMING, 1)
+    m.calculate_symmetry_function_groups(False)
+    m.calculate_atomic_neural_networks(True)
+    assert m.kernel_time("sf64")[1] == 0
+    m.calculate_symmetry_function_groups(True)
+    assert m.kernel_time("sf64")[1] == 1
+    m.calculate_forces()
+    assert m.kernel_time("sf64")[1] == 1
+    o = Oracle(d)
+    o.set_structure(pos, elem, box)
+    o.predict(PULL, BRUTE)
+    assert np.abs(m.forces() - o.forces()).max() <= 1e-10  # the plain form's against the oracle
