@@ -17,7 +17,7 @@ def say(*a):
     print(*a, flush=True)
 
 
-def model(kind, directory):
+def model(kind, directory, linear=False):
     lines = []
     for c in ("H", "O"):
         lines += ["%s 20 %s %s p2a" % (c, n, w) for n in "HO" for w in ("-6.0 6.0", "0.5 4.0", "0.0 5.0")]
@@ -40,7 +40,11 @@ def model(kind, directory):
     # weighted functions run to 10^4: a thousandth of them for the networks
     top = 1000.0 if kind == "weighted" else 1.0
     rows = [(e + 1, k + 1, 0.0, top, 0.0, 1.0) for e in range(2) for k in range(len(sfs[e]))]
-    synth.write_model(directory, ("H", "O"), lines, (10, 10), ("t", "t", "l"), rows)
+    if linear:  # a quarter of each function's value: exact in either precision
+        weights = {c: np.concatenate([np.full(len(f), 0.25), [0.0, 1.0, 0.0]]) for c, f in zip("HO", sfs)}
+        synth.write_model(directory, ("H", "O"), lines, (1,), ("l", "l"), rows, weights=weights)
+    else:
+        synth.write_model(directory, ("H", "O"), lines, (10, 10), ("t", "t", "l"), rows)
     return directory
 
 
@@ -120,3 +124,39 @@ def test_force_sums_in_64_bits(tmp_path):
     err = np.abs(F[n2p2_amd.MIXED] / F[n2p2_amd.PLAIN_FP64] - 1.0)
     say("  rel errors", " ".join("%.1e" % x for x in err))
     assert err.max() <= 3e-7
+
+
+@pytest.mark.parametrize("n", [250, 280, 400, 440])
+@pytest.mark.parametrize("kind", ["full", "unfactored", "weighted"])
+def test_factored_and_members_by_list_length(kind, n, tmp_path):
+    """The factored kernel stages up to 256 neighbours in FP64 and 416 in FP32
+    where it takes derivatives (the plain form by the list's capacity, here
+    the atoms in 32s); longer lists go member by member.  Atoms that are all
+    each other's neighbours, on both sides of either limit, with the bounds of
+    test_factored_against_members: the mixed form's networks, linear with exact
+    weights, add one rounding of 6e-8 to the functions' dozen."""
+    say("case: compact functions, %s, %d atoms within the cutoff" % (kind, n))
+    d = model(kind, str(tmp_path / "m"), linear=True)
+    rng = np.random.default_rng(n)
+    pos = np.zeros((1, 3))
+    while len(pos) < n:
+        p = rng.uniform(-2.9, 2.9, 3)
+        if np.linalg.norm(p) < 2.9 and ((pos - p) ** 2).sum(1).min() > 0.16:
+            pos = np.vstack([pos, p])
+    elem = (np.arange(n) % 3 == 0).astype(np.int32)
+    vE, vF = rng.normal(size=1), rng.normal(size=pos.shape)
+    got = {}
+    for name, stored, precision in (("stored", 1, n2p2_amd.PLAIN_FP64), ("plain", 0, n2p2_amd.PLAIN_FP64),
+                                    ("mixed", 0, n2p2_amd.MIXED)):
+        m = n2p2_amd.Mode(d)
+        m.set_option(n2p2_amd.OPT_PLAIN_FORCES, stored)
+        m.set_structures(pos, elem)
+        m.evaluate(precision, forces=True)
+        got[name] = [m.G(), m.energies(), m.forces(), m.weight_vjp(vE, vF, precision)]
+    assert m.neighbors()[0].max() == n - 1
+    for name, tol in (("plain", (1e-11,) * 4), ("mixed", (2e-6,) * 4)):
+        for what, a, b, t in zip(("G", "energies", "forces", "rows"), got[name], got["stored"], tol):
+            err = float(np.abs(a - b).max() / np.abs(b).max())
+            say("  %s: max rel %.2e" % (name + " " + what, err))
+            assert np.isfinite(a).all()
+            assert err <= t

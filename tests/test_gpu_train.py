@@ -230,10 +230,10 @@ def test_weight_vjp_wide_network(wide_case, precision):
 
 @pytest.mark.parametrize("precision", [n2p2_amd.PLAIN_FP64, n2p2_amd.MIXED])
 def test_loss_gradient_wide_network(precision, tmp_path):
-    """nnpx_loss_gradient (one summed gradient) with the 50-100-100-1 network
-    whose FP64 connection gradient exceeds the LDS accumulator: every atom's
-    connections go into one row through the global-atomic variant; three
-    66-78 atom water structures against the oracle's loss gradient."""
+    """nnpx_loss_gradient (one summed gradient) with the 50-100-100-1 network,
+    whose FP64 connection sums do not fit the LDS: each block adds its tiles'
+    sums to its own row in device memory, and the weights are read from there;
+    three 66-78 atom water structures against the oracle's loss gradient."""
     d = synth.water_model(str(tmp_path / "wide"), hidden=(100, 100))
     t = synth.water_model(str(tmp_path / "wide_teacher"), hidden=(100, 100), seed=synth.SEED_TEACHER)
     say("case: loss gradient, 50-100-100-1 network, 3 water structures, precision %d" % precision)
@@ -257,13 +257,13 @@ def test_loss_gradient_wide_network(precision, tmp_path):
 @pytest.mark.parametrize("per_block", [1, 5, 16, 32])
 @pytest.mark.parametrize("precision", [n2p2_amd.PLAIN_FP64, n2p2_amd.MIXED])
 def test_gradient_tiles(models, precision, per_block):
-    """The gradient kernel's tiles of atoms: 352 uneven structures (15 to 48
+    """The gradient kernel's tiles of atoms: 352 uneven structures (15 to 45
     atoms, so a tile of 16 holds parts of several and its last one is partly
     filled) as 32 copies of 11, against the rows of the 11 alone (tiles of a
     few atoms, pinned to the oracle above).  The terms are equal and only the
-    order of the FP64 sums differs: 1e-12 relative covers their 352 x 48
+    order of the FP64 sums differs: 1e-12 relative covers their 352 x 45
     terms.  The mixed form's few atoms are evaluated by four waves each and
-    the many by two, so their FP32 term sums also run in another order: terms
+    the many by one, so their FP32 term sums also run in another order: terms
     of 6e-8 rounding, sums of up to a hundred of them per lane before
     compensation, below 1e-5 of the largest row."""
     say("case: gradient tiles, 352 structures, %d atoms per block, precision %d" % (per_block, precision))
@@ -330,3 +330,45 @@ def test_tangent_sums_in_64_bits(tmp_path):
     # the network pass takes the tangent rounded to FP32 (6e-8 each side); a
     # term has a dozen FP32 factors, two of them hardware sines and cosines
     assert worst[0] <= 1.2e-7 and worst[1] <= 2e-6
+
+
+@pytest.mark.parametrize("members", [False, True])
+def test_tangent_waves(models, members, tmp_path):
+    """The mixed tangent with four, two and one wave per atom: 330 atoms in 11
+    structures, 1,320 in four and 4,290 in thirteen copies of them, on the
+    power path and with a third exponent, which takes the member path.  Rows of
+    the copies against those of the 11 (equal FP32 terms; their sums, in FP64 or
+    compensated, in another order: 1e-6 of the largest row, with the network
+    pass in FP32) and those against the plain form's (the networks' FP32 pass
+    and the functions' FP32 terms: 2e-5)."""
+    say("case: tangent on four, two and one wave per atom, %s path" % ("member" if members else "power"))
+    d = models[0]
+    if members:
+        lines = [x for x in synth.water_sf_lines() if " 3 " not in x]
+        lines += ["%s 3 %s %g %g %g 6.35" % (c, p, eta, lam, z) for c in "HO" for p in ("H H", "H O", "O O")
+                  for eta, lam, z in ((0.001, 1, 1), (0.01, -1, 3), (0.03, 1, 4), (0.1, -1, 16))]
+        pos, elem, box = synth.water_box(3)
+        rows = synth.scaling_rows(synth.sorted_sfs(lines, ("H", "O")), pos, elem, box)
+        d = str(tmp_path / "members")
+        synth.write_model(d, ("H", "O"), lines, (25, 25), ("t", "t", "l"), rows)
+    parts = [synth.water_set(1, k, k, seed=synth.SEED_WATERSET + k) for k in range(5, 16)]
+    pos, elem, boxes = (np.concatenate([p[k] for p in parts]) for k in range(3))
+    off = np.concatenate([[0], np.cumsum([len(p[1]) for p in parts])])
+    rng = np.random.default_rng(53)
+    vE, vF = rng.normal(size=11), rng.normal(size=(len(elem), 3))
+    m = n2p2_amd.Mode(d)
+    few = None
+    for n in (1, 4, 13):
+        m.set_structures(np.tile(pos, (n, 1)), np.tile(elem, n), np.tile(boxes, (n, 1, 1)),
+                         np.concatenate([[0], np.cumsum(np.tile(np.diff(off), n))]))
+        rows = m.weight_vjp(np.tile(vE, n), np.tile(vF, (n, 1)), n2p2_amd.MIXED)
+        if few is None:
+            few = rows
+            plain = m.weight_vjp(vE, vF, n2p2_amd.PLAIN_FP64)
+            top = float(np.abs(plain).max())
+            say("  four waves against the plain form: %.2e" % (float(np.abs(few - plain).max()) / top))
+            assert np.abs(few - plain).max() <= 2e-5 * top
+        else:
+            err = float(np.abs(rows - np.tile(few, (n, 1))).max()) / top
+            say("  %d atoms against 330: %.2e" % (n * len(elem), err))
+            assert err <= 1e-6
