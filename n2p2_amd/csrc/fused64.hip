@@ -32,14 +32,16 @@
 // Neighbour sums are pushed to the force array with FP64 device atomics;
 // the pull form drops the atom's own periodic images (Mode.cpp:1957).
 //
-// Bound by FP64 instruction issue, which needs four waves per SIMD: one wave
-// per atom left 2.5 (its 12 KB of staging fills the LDS first), two share it;
-// the walks' registers allow four once the other cutoff types' code and the
-// series' coefficients are out of them (cutoff_fdf64, in_place).  Water of
-// 12,288 atoms, two eta, 30 angular functions per element: values 502 -> 355
-// us, forces 657 -> 553 us (606 with one wave per atom, 773 with four: the
-// waves' last buffers are filled less).  5,100 atoms: the tangent 263 us and
-// 211 us of values where storing dG/dr took 2,694 us and its tangent 152 us.
+// Bound by FP64 instruction issue (75% of the time in the values, 58% in the
+// forces), which wants four waves per SIMD: one wave per atom left 2.1 and 1.8
+// (its 12 KB of staging fills the LDS first), two that share it 4.2 and 3.3; the
+// registers allow five and four once the other cutoff types' code and the
+// series' coefficients are out of the walks (cutoff_fdf64, in_place; the forces
+// still spill 39 at their 128).  Water of 12,288 atoms, two eta, 30 angular
+// functions per element: values 506 -> 368 us, forces 665 -> 580 us between the
+// bench line's markers (with four waves the forces take 40% more: the waves'
+// last buffers are filled less).  5,100 atoms: the tangent 255 us and 212 us of
+// values where storing dG/dr took 2,694 us and its tangent 152 us.
 #include <string>
 #include <type_traits>
 
@@ -51,8 +53,8 @@
 namespace nnpx {
 namespace {
 
-// Pairs in a wave's buffer, fewer where LDS is short (water, 12,288 atoms:
-// values 355 us at 256 pairs, 377 at 384; forces 553, 551).
+// Pairs in a wave's buffer, fewer where LDS is short (water, 12,288 atoms,
+// kernel trace: values 355 us at 256 pairs, 377 at 384; forces 553, 551).
 constexpr int kWalk64 = 256;
 constexpr int kMinWalk64 = 128;  // ... at least
 constexpr size_t kLds64 = 65536;

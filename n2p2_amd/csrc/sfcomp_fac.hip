@@ -26,9 +26,11 @@
 // in registers over the run, partner k's force goes through LDS FP64 atomics.
 // Radial members: a wave each (values, tangent); threads own neighbours
 // (force).
-//   Bound by instruction issue at two or three waves per SIMD (294 vector
-// instructions per triplet for 54 values, 480 for their forces; 64 FP64 sums
-// take 128 registers).  184 functions and 185 neighbours per atom, 1,152 atoms,
+//   Bound by instruction issue (294 vector instructions per triplet for 54
+// values, 480 for their forces) with few waves to hide the rest: the registers
+// allow two per SIMD for the values (64 FP64 sums take 128) and three for the
+// forces; 1,152 atoms, 4.5 blocks per CU, keep 1.3 and 1.8 resident, which issue
+// 43% and 63% of the time.  For those, 184 functions and 185 neighbours each,
 // FP32 terms: values 4,344 us member by member -> 335 us, forces 4,872 -> 377
 // us (647 and 639 with a switch over the cores and a window test per function
 // in the walk; forces 370 with a run's sums in FP32, which cost up to 8e-7 of a
