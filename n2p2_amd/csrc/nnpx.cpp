@@ -797,6 +797,17 @@ void settle(nnpx_ctx* c)
     c->settled = true;
 }
 
+// A structure set that is refused or cannot be copied after its atom count was
+// taken leaves none: kernels must not run that many atoms on other buffers.
+struct Taking {
+    nnpx_ctx* c;
+    bool done = false;
+    ~Taking()
+    {
+        if (!done) c->N = c->S = 0;
+    }
+};
+
 // Structures of nnpx_set_structures (copied to device buffers; the first
 // neighbour build sizes the list capacity).
 void set_structures(nnpx_ctx* c, int ns, const int64_t* off, const double* pos, const int* elem, const double* box,
@@ -820,6 +831,7 @@ void set_structures(nnpx_ctx* c, int ns, const int64_t* off, const double* pos, 
     for (int64_t i = 0; i < N; ++i)
         if (elem[i] < 0 || elem[i] >= c->hm.t.nelem) fail(NNPX_ERR_RANGE, "element index out of range");
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    Taking taking{c};
     c->N = (int)N;
     c->S = ns;
     c->atom_off.assign(off, off + ns + 1);
@@ -853,6 +865,7 @@ void set_structures(nnpx_ctx* c, int ns, const int64_t* off, const double* pos, 
                {"st", c->st_host.data(), sizeof(StructT) * ns},
                {"elem_atoms", atoms.data(), sizeof(int) * N},
                {"atom_off", off32.data(), sizeof(int) * (ns + 1)}});
+    taking.done = true;
     c->cap = estimate_cap(c);
     c->nbr_valid = false;
     invalidate(c);
@@ -1270,6 +1283,7 @@ nnpx_status nnpx_set_neighbors_external(nnpx_ctx* c, int nlocal, const int* elem
         c->skin = 0.0;
         c->external = true;
         c->list_fresh = false;
+        Taking taking{c};
         c->ntotal = ntotal;
         c->N = nlocal;
         c->S = 1;
@@ -1318,6 +1332,7 @@ nnpx_status nnpx_set_neighbors_external(nnpx_ctx* c, int nlocal, const int* elem
         hip_check(hipGetLastError(), "spread");
         fill_int(buf<int>(c, "flags", 4), 0, 4, c->stream);
         buf<int>(c, "nb_rev", slots);
+        taking.done = true;
         invalidate(c);
         c->nbr_valid = true;
         c->rev_valid = true;

@@ -147,3 +147,26 @@ def test_new_weights(water, precision):
     assert np.abs(half[0] - plain[0]).max() <= 6e-5 * np.abs(plain[0]).max()
     m.set_weights(w)
     same(result(m, precision), before, precision)
+
+
+def test_refused_structures_leave_none(tmp_path):
+    """A set refused for its box, of more atoms than the last one, leaves the
+    context without structures: nothing evaluates that many atoms on the last
+    set's buffers.  The next set is taken as ever."""
+    d = synth.water_model(str(tmp_path / "water"))
+    pos, elem, box = synth.water_box(2)
+    m = n2p2_amd.Mode(d)
+    m.set_structures(pos, elem, box[None])
+    m.evaluate(n2p2_amd.PLAIN_FP64, forces=True)
+    E = m.energies()[0]
+    big, elem2, box2 = synth.water_box(4)
+    flat = box2.copy()
+    flat[2] = flat[1]
+    with pytest.raises(n2p2_amd.NNPError, match="singular box"):
+        m.set_structures(big, elem2, flat[None])
+    for call in (m.evaluate, m.calculate_neighbor_list):
+        with pytest.raises(n2p2_amd.NNPError, match="no structures set"):
+            call()
+    m.set_structures(pos, elem, box[None])
+    m.evaluate(n2p2_amd.PLAIN_FP64, forces=True)
+    assert m.energies()[0] == E
