@@ -37,7 +37,7 @@
 // (its 12 KB of staging fills the LDS first), two that share it 4.2 and 3.3; the
 // registers allow five and four once the other cutoff types' code and the
 // series' coefficients are out of the walks (cutoff_fdf64, in_place; the forces
-// still spill 39 at their 128).  Water of 12,288 atoms, two eta, 30 angular
+// still spill 34 at their 128).  Water of 12,288 atoms, two eta, 30 angular
 // functions per element: values 506 -> 368 us, forces 665 -> 580 us between the
 // bench line's markers (with four waves the forces take 40% more: the waves'
 // last buffers are filled less).  5,100 atoms: the tangent 255 us and 212 us of

@@ -88,7 +88,7 @@ __device__ inline int stage_by_element(const ModelT* __restrict__ M, const SysVi
     int next = incl - tot, seen = 0;
     if (wv == 0 && lane <= ne) eoff[lane] = min(lane < ne ? next : total, capL);
     auto place = [&](int p, const Entry& x) {
-        for (; seen < min(p, kLast); ++seen)
+        for (; seen < p; ++seen)
             if (lane < ne) next += cnt[seen * kMaxElem + lane];
         int pos = -1;
         for (int e = 0; e < ne; ++e) {
@@ -97,14 +97,23 @@ __device__ inline int stage_by_element(const ModelT* __restrict__ M, const SysVi
             if (x.el == e)
                 pos = at + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                           __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-            if (p >= kLast && lane == e) next += __popcll(m);  // for the passes that share its row
         }
         if (pos >= 0 && pos < capL) store(pos, p * kWave + lane, x.dr, x.d, x.el);
     };
 #pragma unroll
     for (int q = 0; q < kKeep; ++q)
         if (wv + q * W < npass) place(wv + q * W, keep[q]);
-    for (int p = wv + kKeep * W; p < mine; p += p < kLast ? W : 1) place(p, entry(p));
+    for (int p = wv + kKeep * W; p < mine; p += p < kLast ? W : 1) {
+        const Entry x = entry(p);
+        place(p, x);
+        if (p >= kLast) {  // for the passes that share its row
+            for (int e = 0; e < ne; ++e) {
+                const int c = __popcll(__ballot(x.el == e));
+                if (lane == e) next += c;
+            }
+            seen = p + 1;
+        }
+    }
     if (threadIdx.x == 0) {
         if (total > capL) atomicOr(&s.flags[0], 4);
         if (total > __hip_atomic_load(&s.flags[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
